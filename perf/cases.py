@@ -688,7 +688,7 @@ def tolerance(case):
     if case["kind"] == "sampler":
         return {"rel": 1e-6, "max": 1e-4, "differ": 0.01}
     if case["kind"] == "model":
-        return {"rel": 0.03, "max": 1.0}
+        return {"rel": 0.03, "max": 0.5}
     if case["type"] == "f16":
         return {"rel": 2e-4, "max": 0.02, "differ": 0.01}
     if case["kind"] == "head":
