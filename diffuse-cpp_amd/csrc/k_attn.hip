@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 // One workgroup per (32-row tile, head of Q|K|V), head size HD.  Q and K heads: wave
 // w rotates rows w, w+4, .., w+28 of the tile; HD/8 lanes share a row, each rotating
@@ -137,225 +138,7 @@ __device__ __forceinline__ double4v mfma_f64(double a, double b, double4v c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Matrix-core attention: one head and 16 query rows per workgroup of NW waves.
-// Phase 1: S = Q K^T on the f64 MFMA; each wave takes key tiles of 16 (t = wave + NW j),
-// the next tiles' keys are loaded while the current one multiplies (KR-slot ring), and
-// the head dims are reduced in four independent accumulation chains (dims 16s+4g+c to
-// MFMA c for step s), added at the end as (c0 + c1) + (c2 + c3).
-// Phase 2: softmax, one wave per row, scores resident in LDS.
-// Phase 3: O = P V on the f64 MFMA; wave w owns head-dim columns 16w+16 NW ct+(0..15),
-// keys are the reduction: lane group g supplies keys 16s+4g+c to MFMA c, read as one
-// float4 of the transposed value cache, four key steps ahead; two chains (c even / odd).
-// Every output element's sums are the same for every NW: the wave count only decides which
-// wave computes them.  With eight waves (and at most 128 VGPRs) two workgroups share a CU
-// at four waves per SIMD, and each workgroup finishes in about half the time of four waves.
-// Workgroups are numbered so that all query tiles of head h run on XCD h % 8.  With vs = 2
-// (grids that leave CUs idle) each query tile runs as two workgroups that both form the scores
-// and probabilities and take half of the value columns each (phase 3 on half the waves): the
-// same operations for every output element, so the same bits.
-template <int HD, int KR, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 1)))
-k_attn_mfma(const float * __restrict__ q, const float * __restrict__ kc, const float * __restrict__ vt, int64_t v_ld,
-            int M, int n_keys, int H, int Hkv, int sstride, int q_tiles, int q_pos0, int window,
-            float * __restrict__ out, int vs) {
-#pragma clang fp contract(off)
-    extern __shared__ float S[];       // [16][sstride] scores, then probabilities
-    constexpr int SS = HD / 16;        // reduction steps of 16 head dims
-    constexpr int CT = HD / (16 * NW); // phase-3 column tiles per wave
-    static_assert(CT >= 1 && CT * 16 * NW == HD, "head dims split evenly over the waves");
-    const int L = blockIdx.x, xcd = L & 7, j = L >> 3, slots = q_tiles * vs;
-    const int h = 8 * (j / slots) + xcd, qt = (j % slots) / vs, part = (j % slots) % vs;
-    if (h >= H) return;
-    const int kvh = h / (H / Hkv);
-    const int q0 = qt * 16;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const bool pv = (wv * vs) / NW == part;   // this wave's value columns are this workgroup's
-    const int li = lane & 15, lg = lane >> 4;
-    const int64_t kvstride = (int64_t)Hkv * HD;
-    const float scale = 1.0f / sqrtf((float)HD);
-    const int ntiles = (n_keys + 15) >> 4;
-
-    // ---- phase 1
-    float4 qf[SS];
-    {
-        const int row = q0 + li;
-        const float * qr = q + ((int64_t)min(row, M - 1) * H + h) * HD + 4 * lg;
-#pragma unroll
-        for (int s = 0; s < SS; s++) qf[s] = ld4_or0(qr + 16 * s, row < M);
-    }
-    const float * kbase = kc + (int64_t)kvh * HD + 4 * lg;
-    auto load_k = [&](float4 (&kf)[SS], int t) {
-        const int n = 16 * t + li;
-        const float * kr = kbase + (int64_t)min(n, n_keys - 1) * kvstride;
-#pragma unroll
-        for (int s = 0; s < SS; s++) kf[s] = ld4_or0(kr + 16 * s, n < n_keys);
-    };
-    // key tiles t = wv + NW j in a KR-slot register ring, KR - 1 tiles in flight ahead
-    // of the one being multiplied (slot roles fixed by unrolling, so no copies)
-    float4 kr[KR][SS];
-    auto tile = [&](float4 (&kf)[SS], int t) __attribute__((always_inline)) {
-        double4v a[4] = {0.0, 0.0, 0.0, 0.0};      // four independent chains: MFMA c of each step
-#pragma unroll
-        for (int s = 0; s < SS; s++) {
-            const float kb[4] = {kf[s].x, kf[s].y, kf[s].z, kf[s].w};
-            float qa[4] = {qf[s].x, qf[s].y, qf[s].z, qf[s].w};
-            if constexpr (NW == 8) {
-                // converted to double at each use, not once for the whole kernel: the 64
-                // VGPRs of a hoisted double copy do not fit four waves per SIMD
-#pragma unroll
-                for (int c = 0; c < 4; c++) asm volatile("" : "+v"(qa[c]));
-            }
-#pragma unroll
-            for (int c = 0; c < 4; c++) a[c] = mfma_f64((double)qa[c], (double)kb[c], a[c]);
-        }
-        const double4v acc = (a[0] + a[1]) + (a[2] + a[3]);
-        const int n = 16 * t + li;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            // masked keys score -inf: weight exactly 0 in the sums below
-            const key_range kr = row_keys(q0 + lg + 4 * i, M, n_keys, q_pos0, window);
-            S[(lg + 4 * i) * sstride + n] = n >= kr.lo && n <= kr.hi ? (float)acc[i] * scale : -INFINITY;
-        }
-    };
-#pragma unroll
-    for (int u = 0; u < KR; u++)
-        if (wv + NW * u < ntiles) load_k(kr[u], wv + NW * u);
-    for (int t0 = wv; t0 < ntiles; t0 += NW * KR) {
-#pragma unroll
-        for (int u = 0; u < KR; u++) {
-            const int t = t0 + NW * u;
-            if (t < ntiles) {
-                tile(kr[u], t);
-                if (t + NW * KR < ntiles) load_k(kr[u], t + NW * KR);
-            }
-        }
-    }
-    __syncthreads();
-
-    // The first value steps of phase 3 are loaded here, so that their latency passes under the
-    // softmax.  Value column of this lane for column tile ct: 16*wv + 16*NW*ct + li; keys
-    // 16s+4g..+3.
-    const float * vb = vt + ((int64_t)kvh * HD + 16 * wv + li) * v_ld + 4 * lg;
-    auto load_v = [&](float4 (&vf)[CT], int s) {
-        const int n = 16 * s + 4 * lg;                 // first of this lane's 4 keys
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) {
-            const float * p = vb + (int64_t)16 * NW * ct * v_ld + 16 * min(s, ntiles - 1);
-            // v_ld and n are multiples of 4 and n_keys <= v_ld: the load stays in the row;
-            // keys past the end of the sequence count as 0
-            const f32x4 v = *(const f32x4 *)p;
-            vf[ct] = make_float4(n < n_keys ? v.x : 0.0f, n + 1 < n_keys ? v.y : 0.0f, n + 2 < n_keys ? v.z : 0.0f,
-                                 n + 3 < n_keys ? v.w : 0.0f);
-        }
-    };
-    constexpr int PV = 4;                           // value steps in flight
-    float4 vq[PV][CT];
-    if (pv)
-#pragma unroll
-        for (int u = 0; u < PV; u++) load_v(vq[u], u);
-
-    // ---- phase 2: the wave's RPW rows (wv, wv + NW, ..) together, four keys per lane and
-    // row at a time, so that RPW * 4 exponentials and the rows' reductions are in flight at
-    // once.  Each lane sums its keys lane, lane + 64, .. in increasing order and the lanes
-    // are added by the xor butterfly, one row as another.
-    {
-        constexpr int RPW = 16 / NW;
-        float mx[RPW];
-#pragma unroll
-        for (int q = 0; q < RPW; q++) mx[q] = -INFINITY;
-        for (int n0 = lane; n0 < n_keys; n0 += 256)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int n = n0 + 64 * u;
-#pragma unroll
-                for (int q = 0; q < RPW; q++)
-                    if (n < n_keys) mx[q] = fmaxf(mx[q], S[(wv + NW * q) * sstride + n]);
-            }
-#pragma unroll
-        for (int q = 0; q < RPW; q++) mx[q] = wave_max(mx[q]);
-        double sum[RPW];
-#pragma unroll
-        for (int q = 0; q < RPW; q++) sum[q] = 0.0;
-        for (int n0 = lane; n0 < n_keys; n0 += 256) {
-            float e[RPW][4];
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int q = 0; q < RPW; q++) {
-                    const int n = min(n0 + 64 * u, n_keys - 1);
-                    e[q][u] = (float)exp((double)(S[(wv + NW * q) * sstride + n] - mx[q]));
-                }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int n = n0 + 64 * u;
-                if (n < n_keys)
-#pragma unroll
-                    for (int q = 0; q < RPW; q++) {
-                        S[(wv + NW * q) * sstride + n] = e[q][u];
-                        sum[q] += (double)e[q][u];
-                    }
-            }
-        }
-        float inv[RPW];
-#pragma unroll
-        for (int q = 0; q < RPW; q++) {
-            sum[q] = wave_sum_d(sum[q]);
-            inv[q] = (float)(1.0 / sum[q]);
-        }
-        for (int n0 = lane; n0 < n_keys; n0 += 256)
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int n = n0 + 64 * u;
-                if (n < n_keys)
-#pragma unroll
-                    for (int q = 0; q < RPW; q++) S[(wv + NW * q) * sstride + n] *= inv[q];
-            }
-#pragma unroll
-        for (int q = 0; q < RPW; q++)
-            for (int n = n_keys + lane; n < 16 * ntiles; n += 64) S[(wv + NW * q) * sstride + n] = 0.0f;
-    }
-    __syncthreads();
-
-    // ---- phase 3
-    if (!pv) return;
-    double4v o[CT][2];                              // chains: column tile x MFMA parity
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) o[ct][0] = o[ct][1] = 0.0;
-    for (int s0 = 0; s0 < ntiles; s0 += PV) {
-#pragma unroll
-        for (int u = 0; u < PV; u++) {
-            const int s = s0 + u;
-            if (s < ntiles) {
-                float4 vcur[CT];
-#pragma unroll
-                for (int ct = 0; ct < CT; ct++) vcur[ct] = vq[u][ct];
-                load_v(vq[u], s + PV);
-                const float4 pf = *(const float4 *)(S + li * sstride + 16 * s + 4 * lg);
-                const float pa[4] = {pf.x, pf.y, pf.z, pf.w};
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const double a = (double)pa[c];
-#pragma unroll
-                    for (int ct = 0; ct < CT; ct++) {
-                        const float vv[4] = {vcur[ct].x, vcur[ct].y, vcur[ct].z, vcur[ct].w};
-                        o[ct][c & 1] = mfma_f64(a, (double)vv[c], o[ct][c & 1]);
-                    }
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int row = q0 + lg + 4 * i;
-        if (row >= M) continue;
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++)
-            out[(int64_t)row * H * HD + (int64_t)h * HD + 16 * wv + 16 * NW * ct + li] =
-                (float)(o[ct][0][i] + o[ct][1][i]);
-    }
-}
-
-// ---- split-bf16 matrix-core attention (the default)
+// ---- split-bf16 matrix-core attention (DFX_ATTN_SPLIT_BF16)
 //
 // Every f32 operand x is split into three bf16 parts, x = hi + mid + lo with
 // hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid) (each rounded to nearest,
@@ -588,9 +371,9 @@ __global__ void __launch_bounds__(256, 2) k_attn_split(const float * __restrict_
     }
 }
 
-// Exact form for any key count: the score rows are not kept (they need not fit the LDS);
+// Exact form for any key count: the score rows are not kept;
 // each 16-key score tile is recomputed in three passes over the keys, with the same
-// products, sums and rounding as k_attn_mfma's phase 1, so every pass sees the same scores:
+// products, sums and rounding as k_attn_keep's phase 1, so every pass sees the same scores:
 //   pass 1: row maxima;
 //   pass 2: e = exp(s - max) (correctly rounded), sums in double, inv = (float)(1 / sum);
 //   pass 3: per block of 64 keys, the four waves' probability tiles p = e * inv go through
@@ -617,7 +400,10 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
     const int li = lane & 15, lg = lane >> 4;
     const int64_t kvstride = (int64_t)Hkv * HD;
     const float scale = 1.0f / sqrtf((float)HD);
-    const int ntiles = (n_keys + 15) >> 4, nblocks = (ntiles + 3) >> 2;
+    const int ntiles = (n_keys + 15) >> 4;
+    // key tiles that some row of the query tile sees
+    const int t0 = row_keys(q0, M, n_keys, q_pos0, window).lo >> 4;
+    const int t1 = (row_keys(q0 + 15, M, n_keys, q_pos0, window).hi >> 4) + 1;
 
     float4 qf[SS];
     {
@@ -652,7 +438,7 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
 
     // ---- pass 1: row maxima (lane: rows lg + 4i)
     float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    for (int t = wv; t < ntiles; t += 4) {
+    for (int t = t0 + wv; t < t1; t += 4) {
         float sc[4];
         scores(t, sc);
 #pragma unroll
@@ -672,7 +458,7 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
 
     // ---- pass 2: sums of e = exp(s - max) in double
     double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int t = wv; t < ntiles; t += 4) {
+    for (int t = t0 + wv; t < t1; t += 4) {
         float sc[4];
         scores(t, sc);
 #pragma unroll
@@ -696,7 +482,7 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) o[ct][0] = o[ct][1] = 0.0;
     const float * vb = vt + ((int64_t)kvh * HD + 16 * wv + li) * v_ld;
-    for (int b = 0; b < nblocks; b++) {
+    for (int b = t0 >> 2; b < (t1 + 3) >> 2; b++) {
         const int t = 4 * b + wv;
         float sc[4];
         scores(min(t, ntiles - 1), sc);
@@ -742,86 +528,298 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
     }
 }
 
-// Few query rows (autoregressive decoding: one row per token): one workgroup of 4 waves per
-// (row, head) instead of a 16-row tile per head.  Scores: 16 lanes per key, each adding the
-// products of its HD/16 dimensions in f64 (f32 x f32 products are exact there), the 16 partial
-// sums added by an xor butterfly, rounded to float and scaled; 16 keys per round.  Softmax as the
-// oracle: max, e = (float)exp((double)(s - max)), sum in double, p = e * (float)(1 / sum).
-// Output: HD dimensions x 256/HD key ranges per workgroup, each range summed in f64 in key order
-// (16-byte loads of the transposed value cache), the ranges' f64 sums added in order, rounded to
-// float once.  Only the f64 summation order differs from the oracle's (as in the matrix-core
-// kernels): a float result differs where two orders straddle a rounding boundary.
-// At most ROWS_MAX_KEYS visible keys per row.
-#define ROWS_MAX_KEYS 1024
-template <int HD>
-__global__ void __launch_bounds__(256) k_attn_rows(const float * __restrict__ q, const float * __restrict__ kc,
-                                                   const float * __restrict__ vt, int64_t v_ld, int M, int n_keys,
-                                                   int H, int Hkv, int q_pos0, int window, float * __restrict__ out) {
+// Exact matrix-core attention, the scores kept in registers: up to 128 * NT visible keys, one head
+// and 16 query rows per workgroup of eight waves; wave w takes the 16-key tiles t0 + w + 8j, j < NT.
+// Phase 1: S^T = K Q^T on the f64 MFMA: lane (li, lg) holds query li's scores of four keys per
+// tile (the keys are assigned to the tile's rows so that these are keys 4 lg .. 4 lg + 3), the
+// query as doubles in LDS, half a tile of keys (64 dims) loaded under the other half's MFMAs; the
+// head dims in four independent chains (dims 16s + 4g + c to chain c), added (c0 + c1) + (c2 + c3).
+// Phase 2: softmax in registers: a lane's keys, the four lane groups, the waves (through LDS).
+// Phase 3: O^T = V^T P^T over the wave's own keys: a lane's four probabilities are the B operands
+// of four MFMAs as they are, the A operands one 16-byte load of the transposed value cache per
+// 16 value columns; the waves' f64 sums are added in a fixed order through LDS.
+// Key tiles that no row of the query tile sees are not visited.
+// Bound by the f64 matrix cores (62 TFLOP/s measured on a large product): 4096 keys, 512 causal
+// rows of 28 heads 620 us (floor 455) against 1704 when the scores were recomputed in three
+// passes; 768 keys and rows of 32 heads 192 us (floor 156) against 222 with scores in LDS, whose
+// softmax read and wrote them three times; 288 by 288 46 against 52.  WPE waves per SIMD: 2 (one
+// workgroup per CU, 256 VGPRs) or 4 (two, half of the partial outputs in LDS at a time).
+template <int HD, int NT, int WPE>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+k_attn_keep(const float * __restrict__ q, const float * __restrict__ kc, const float * __restrict__ vt, int64_t v_ld,
+            int M, int n_keys, int H, int Hkv, int q_tiles, int q_pos0, int window, float * __restrict__ out) {
 #pragma clang fp contract(off)
-    constexpr int DPL = HD / 16;            // dimensions per lane of a key's group
-    constexpr int PARTS = 256 / HD;         // key ranges of the output sums
-    __shared__ float sc[ROWS_MAX_KEYS];
-    __shared__ float red[4];
-    __shared__ double red_d[4];
-    __shared__ double part[PARTS][HD];
+    constexpr int NW = 8, SS = HD / 16, CT = HD / 16;
+    constexpr int RW = WPE == 2 ? NW : NW / 2;       // waves whose partial outputs are in LDS at once
+    __shared__ __attribute__((aligned(16))) double R[RW * HD * 16];   // query [SS][2][64][2], then partial outputs
+    __shared__ float red_f[NW][16];
+    __shared__ double red_d[NW][16];
+    // unit u = (head, query tile), heads of one KV head adjacent; XCD x (= workgroup mod 8) takes
+    // an eighth of the units in order, so that few KV heads share an L2
+    const int units = H * q_tiles, per_xcd = (units + 7) / 8;
+    const int u = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || u >= units) return;
+    const int h = u / q_tiles, q0 = (q_tiles - 1 - u % q_tiles) * 16, kvh = h / (H / Hkv);
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t kvstride = (int64_t)Hkv * HD;
+    const float scale = 1.0f / sqrtf((float)HD);
+    const int t0 = row_keys(q0, M, n_keys, q_pos0, window).lo >> 4;
+    const int t1 = (row_keys(q0 + 15, M, n_keys, q_pos0, window).hi >> 4) + 1;
+    const key_range kr = row_keys(q0 + li, M, n_keys, q_pos0, window);
+
+    const float * kbase = kc + (int64_t)kvh * HD + 4 * lg;
+    const int krow = 4 * (li & 3) + (li >> 2);       // this lane's key of a tile
+    // half a tile's dimensions at a time, the next half loaded under the current one's MFMAs
+    constexpr int HS = SS / 2;
+    f32x4 kf[2][4];
+    auto load_k = [&](auto half, int t) __attribute__((always_inline)) {
+        constexpr int hf = decltype(half)::value;
+        const float * p = kbase + (int64_t)min(16 * t + krow, n_keys - 1) * kvstride + 16 * HS * hf;
+#pragma unroll
+        for (int s = 0; s < HS; s++) kf[hf][s] = *(const f32x4 *)(p + 16 * s);
+    };
+    constexpr std::integral_constant<int, 0> lo{};
+    constexpr std::integral_constant<int, 1> hi{};
+    load_k(lo, min(t0 + wv, t1 - 1));
+
+    // query row li, dims 16s + 4g + c: lane (li, g) of step s, MFMA c
+    for (int e = tid; e < 16 * HD / 4; e += 512) {
+        const int s = e >> 6, l = e & 63, row = q0 + (l & 15);
+        const float4 v = ld4_or0(q + ((int64_t)min(row, M - 1) * H + h) * HD + 16 * s + 4 * (l >> 4), row < M);
+        double * d = R + (size_t)s * 256 + 2 * l;
+        d[0] = (double)v.x; d[1] = (double)v.y;
+        d[128] = (double)v.z; d[129] = (double)v.w;
+    }
+    __syncthreads();
+
+    // ---- phase 1
+    auto mul_k = [&](auto half, double4v (&a)[4]) __attribute__((always_inline)) {
+        constexpr int hf = decltype(half)::value;
+#pragma unroll
+        for (int s = 0; s < HS; s++) {
+            const double2 * qd = (const double2 *)(R + (size_t)(HS * hf + s) * 256) + lane;
+            const double2 q01 = qd[0], q23 = qd[64];
+            const f32x4 kv = kf[hf][s];
+            a[0] = mfma_f64((double)kv.x, q01.x, a[0]);
+            a[1] = mfma_f64((double)kv.y, q01.y, a[1]);
+            a[2] = mfma_f64((double)kv.z, q23.x, a[2]);
+            a[3] = mfma_f64((double)kv.w, q23.y, a[3]);
+        }
+    };
+    float sc[NT][4];
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int t = t0 + wv + NW * j;
+        if (t < t1) {
+            double4v a[4] = {0.0, 0.0, 0.0, 0.0};
+            load_k(hi, t);
+            mul_k(lo, a);
+            load_k(lo, min(t + NW, t1 - 1));
+            mul_k(hi, a);
+            const double4v acc = (a[0] + a[1]) + (a[2] + a[3]);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int n = 16 * t + 4 * lg + i;
+                sc[j][i] = n >= kr.lo && n <= kr.hi ? (float)acc[i] * scale : -INFINITY;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) sc[j][i] = -INFINITY;
+        }
+    }
+
+    // the first value loads' latency passes under the softmax
+    const float * vb = vt + ((int64_t)kvh * HD + li) * v_ld + 4 * lg;
+    constexpr int HC = CT / 2;
+    f32x4 vf[2][4];
+    auto load_v = [&](auto half, int t) __attribute__((always_inline)) {
+        constexpr int hf = decltype(half)::value;
+#pragma unroll
+        for (int c = 0; c < HC; c++) vf[hf][c] = *(const f32x4 *)(vb + (int64_t)16 * (HC * hf + c) * v_ld + 16 * t);
+    };
+    load_v(lo, min(t0 + wv, t1 - 1));
+
+    // ---- phase 2
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) mx = fmaxf(mx, sc[j][i]);
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    if (lg == 0) red_f[wv][li] = mx;
+    __syncthreads();
+    mx = red_f[0][li];
+#pragma unroll
+    for (int w = 1; w < NW; w++) mx = fmaxf(mx, red_f[w][li]);
+    double sum = 0.0;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+        if (t0 + wv + NW * j < t1)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                sc[j][i] = (float)exp((double)(sc[j][i] - mx));
+                sum += (double)sc[j][i];
+            }
+    sum += __shfl_xor(sum, 16, WAVE);
+    sum += __shfl_xor(sum, 32, WAVE);
+    if (lg == 0) red_d[wv][li] = sum;
+    __syncthreads();
+    sum = red_d[0][li];
+#pragma unroll
+    for (int w = 1; w < NW; w++) sum += red_d[w][li];
+    const float inv = (float)(1.0 / sum);
+
+    // ---- phase 3
+    double4v o[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) o[ct] = 0.0;
+    auto mul_v = [&](auto half, int n, const float (&p)[4]) __attribute__((always_inline)) {
+        constexpr int hf = decltype(half)::value;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c < HC; c++)
+                o[HC * hf + c] = mfma_f64((double)(n + i < n_keys ? vf[hf][c][i] : 0.0f), (double)p[i], o[HC * hf + c]);
+    };
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        const int t = t0 + wv + NW * j;
+        if (t < t1) {
+            const int n = 16 * t + 4 * lg;
+            const float p[4] = {sc[j][0] * inv, sc[j][1] * inv, sc[j][2] * inv, sc[j][3] * inv};
+            load_v(hi, t);
+            mul_v(lo, n, p);
+            load_v(lo, min(t + NW, t1 - 1));
+            mul_v(hi, n, p);
+        }
+    }
+    auto put = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) R[((slot * CT + ct) * 4 + i) * 64 + lane] = o[ct][i];
+    };
+    if constexpr (RW < NW) {                         // waves 0 .. RW-1 add the sums of waves RW .. first
+        if (wv >= RW) put(wv - RW);
+        __syncthreads();
+        if (wv < RW)
+#pragma unroll
+            for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) o[ct][i] += R[((wv * CT + ct) * 4 + i) * 64 + lane];
+        if (wv < RW) put(wv);                        // the slots that this wave alone has just read
+    } else if (wv < t1 - t0) {
+        put(wv);
+    }
+    __syncthreads();
+    for (int e = tid; e < HD * 16; e += 512) {
+        double s = R[e];
+#pragma unroll
+        for (int w = 1; w < RW; w++)
+            if (w < t1 - t0) s += R[w * HD * 16 + e];            // waves that had a tile
+        const int row = q0 + (e & 15), d = 4 * ((e >> 6) & 3) + ((e >> 4) & 3) + 16 * (e >> 8);
+        if (row < M) out[((int64_t)row * H + h) * HD + d] = (float)s;
+    }
+}
+
+// Few query rows (autoregressive decoding: one row per token): one workgroup of HD/8 waves per
+// (row, head) instead of a 16-row tile per head.  Scores: 16 lanes per key, each adding the
+// products of HD/16 dimensions in f64 (f32 x f32 products are exact there), the 16 partial sums
+// added across the lanes, rounded to float and scaled.  Softmax as the oracle: max,
+// e = (float)exp((double)(s - max)), sum in double, p = e * (float)(1 / sum).  Output: wave w takes
+// dimensions 8w .. 8w + 7, eight lanes per dimension reading 32 consecutive keys of its value row
+// (whole cache lines), the first PV such steps requested before the scores; the lanes' f64 sums
+// are added at the end and rounded to float once.  Only the f64 summation order differs from the
+// oracle's (as in the matrix-core kernels): a float result differs where two orders straddle a
+// rounding boundary.  Bound by the latency of its loads and one CU's bandwidth: one row of 28
+// heads 7.4 us over 192 keys, 19.9 over 1024, 73.9 over 4096 (four waves and a thread per output
+// dimension and key range, each lane reading its own value row: 10.2, 33.9; the matrix-core tile
+// 582).
+template <int CTRL> __device__ __forceinline__ double dpp_sum(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, true);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
+    return v + __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
+#define ROWS_MAX_KEYS 32768
+template <int HD>
+__global__ void __launch_bounds__(8 * HD) k_attn_rows(const float * __restrict__ q, const float * __restrict__ kc,
+                                                      const float * __restrict__ vt, int64_t v_ld, int M, int n_keys,
+                                                      int H, int Hkv, int q_pos0, int window,
+                                                      float * __restrict__ out) {
+#pragma clang fp contract(off)
+    constexpr int NT = 8 * HD, NW = HD / 8, G = NT / 16;   // threads, waves, key groups of 16 lanes
+    constexpr int DPL = HD / 16;                           // dimensions per lane of a key's group
+    constexpr int RK = 4, PV = 8;
+    extern __shared__ __attribute__((aligned(16))) float sc[];   // keys k0 .. k0 + 32 * steps - 1
+    __shared__ float red[NW];
+    __shared__ double red_d[NW];
     const int h = blockIdx.x % H, row = blockIdx.x / H;
     const int kvh = h / (H / Hkv);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const key_range kr = row_keys(row, M, n_keys, q_pos0, window);
-    const int nk = kr.hi - kr.lo + 1;
+    const int k0 = kr.lo & ~31, steps = (kr.hi - k0) / 32 + 1;
     const float scale = 1.0f / sqrtf((float)HD);
-    const int sub = lane & 15, grp = (tid >> 4);            // grp: key slot 0..15 of a round
+
+    const int vd = 8 * wv + (lane >> 3), vk = 4 * (lane & 7);    // output work: dimension, keys of a step
+    const float * vr = vt + ((int64_t)kvh * HD + vd) * v_ld;
+    auto load_v = [&](int s) __attribute__((always_inline)) {
+        return *(const f32x4 *)(vr + min(k0 + 32 * s + vk, (int)v_ld - 4));   // v_ld is a multiple of 16
+    };
+    const int sub = lane & 15, grp = tid >> 4;
     float qd[DPL];
     {
-        const float * qr = q + ((int64_t)row * H + h) * HD + DPL * sub;
+        const float * qr = q + ((int64_t)row * H + h) * HD + 4 * sub;
 #pragma unroll
         for (int i = 0; i < DPL; i += 4) {
-            const float4 v = *(const float4 *)(qr + i);
+            const f32x4 v = *(const f32x4 *)(qr + 16 * i);
             qd[i] = v.x; qd[i + 1] = v.y; qd[i + 2] = v.z; qd[i + 3] = v.w;
         }
     }
-    // output work of this thread (used after the softmax): dimension d, key range pt of PARTS
-    // (range borders on multiples of 4 keys); the range's first PV x 4 values are requested now,
-    // so that their latency passes during the scores and the softmax
-    constexpr int PV = 8;
-    const int d = tid % HD, pt = tid / HD;
-    const int per = ((nk + PARTS - 1) / PARTS + 3) & ~3;
-    const int ra = kr.lo + pt * per, rb = min(kr.lo + (pt + 1) * per, kr.hi + 1);
-    const float * vr = vt + ((int64_t)kvh * HD + d) * v_ld;
-    const int pa = (ra + 3) & ~3;                 // first 16-byte aligned key of the range
-    float4 vpre[PV];
-#pragma unroll
-    for (int u = 0; u < PV; u++) vpre[u] = *(const float4 *)(vr + min(pa + 4 * u, (int)(v_ld - 4)));
     const int64_t kvstride = (int64_t)Hkv * HD;
-    float mx = -INFINITY;
-    // RK keys per lane group and round, all their loads issued before any arithmetic (a round
-    // at a time would wait out one memory latency per 16 keys)
-    constexpr int RK = 8;
-    for (int j0 = 0; j0 < nk; j0 += 16 * RK) {
-        float4 kv[RK][DPL / 4];
+    const float * kb = kc + (int64_t)kvh * HD + 4 * sub;
+    f32x4 kv[RK][DPL / 4];
+    auto load_k = [&](int n0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < RK; u++) {
-            const int j = min(j0 + grp + 16 * u, nk - 1);
-            const float * kp = kc + (int64_t)(kr.lo + j) * kvstride + (int64_t)kvh * HD + DPL * sub;
+            const float * kp = kb + (int64_t)min(n0 + grp + G * u, kr.hi) * kvstride;
 #pragma unroll
-            for (int i = 0; i < DPL / 4; i++) kv[u][i] = *(const float4 *)(kp + 4 * i);
+            for (int i = 0; i < DPL / 4; i++) kv[u][i] = *(const f32x4 *)(kp + 64 * i);
         }
+    };
+    load_k(kr.lo);
+    f32x4 vpre[PV];
+#pragma unroll
+    for (int u = 0; u < PV; u++) vpre[u] = load_v(min(u, steps - 1));
+    for (int n = k0 + tid; n < k0 + 32 * steps; n += NT)
+        if (n < kr.lo || n > kr.hi) sc[n - k0] = 0.0f;           // keys of the steps outside the range
+    float mx = -INFINITY;
+    for (int n0 = kr.lo; n0 <= kr.hi; n0 += G * RK) {
+        double acc[RK];
 #pragma unroll
         for (int u = 0; u < RK; u++) {
-            double acc = 0.0;
+            acc[u] = 0.0;
 #pragma unroll
-            for (int i = 0; i < DPL / 4; i++) {
-                acc = acc + (double)kv[u][i].x * (double)qd[4 * i];
-                acc = acc + (double)kv[u][i].y * (double)qd[4 * i + 1];
-                acc = acc + (double)kv[u][i].z * (double)qd[4 * i + 2];
-                acc = acc + (double)kv[u][i].w * (double)qd[4 * i + 3];
-            }
+            for (int i = 0; i < DPL / 4; i++)
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1) acc += __shfl_xor(acc, o, WAVE);
-            const int j = j0 + grp + 16 * u;
-            if (sub == 0 && j < nk) {
-                const float sv = (float)acc * scale;
-                sc[j] = sv;
+                for (int c = 0; c < 4; c++) acc[u] = fma((double)kv[u][i][c], (double)qd[4 * i + c], acc[u]);
+        }
+        if (n0 + G * RK <= kr.hi) load_k(n0 + G * RK);
+#pragma unroll
+        for (int u = 0; u < RK; u++) acc[u] = dpp_sum<0xB1>(acc[u]);
+#pragma unroll
+        for (int u = 0; u < RK; u++) acc[u] = dpp_sum<0x4E>(acc[u]);
+#pragma unroll
+        for (int u = 0; u < RK; u++) acc[u] = dpp_sum<0x141>(acc[u]);
+#pragma unroll
+        for (int u = 0; u < RK; u++) {
+            acc[u] = dpp_sum<0x140>(acc[u]);
+            const int n = n0 + grp + G * u;
+            if (n <= kr.hi) {
+                const float sv = (float)acc[u] * scale;
+                if (sub == 0) sc[n - k0] = sv;
                 mx = fmaxf(mx, sv);
             }
         }
@@ -829,67 +827,39 @@ __global__ void __launch_bounds__(256) k_attn_rows(const float * __restrict__ q,
     mx = wave_max(mx);
     if (lane == 0) red[wv] = mx;
     __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    mx = red[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) mx = fmaxf(mx, red[w]);
     double sum = 0.0;
-    for (int j = tid; j < nk; j += 256) {
-        const float e = (float)exp((double)(sc[j] - mx));
-        sc[j] = e;
+    for (int n = kr.lo + tid; n <= kr.hi; n += NT) {
+        const float e = (float)exp((double)(sc[n - k0] - mx));
+        sc[n - k0] = e;
         sum += (double)e;
     }
     sum = wave_sum_d(sum);
     if (lane == 0) red_d[wv] = sum;
     __syncthreads();
-    const float inv = (float)(1.0 / (((red_d[0] + red_d[1]) + red_d[2]) + red_d[3]));
-    for (int j = tid; j < nk; j += 256) sc[j] = sc[j] * inv;
-    __syncthreads();
-    {
-        double acc = 0.0;
-        int n = ra;
-        for (; n < rb && (n & 3); n++) acc = acc + (double)vr[n] * (double)sc[n - kr.lo];
-        // n == pa here (or the range is done): the prefetched 16-byte groups first
+    sum = red_d[0];
+#pragma unroll
+    for (int w = 1; w < NW; w++) sum += red_d[w];
+    const float inv = (float)(1.0 / sum);
+    double o = 0.0;
+    for (int s0 = 0; s0 < steps; s0 += PV) {
 #pragma unroll
         for (int u = 0; u < PV; u++) {
-            if (n + 4 <= rb) {
-                const float * pp = sc + (n - kr.lo);
-                acc = acc + (double)vpre[u].x * (double)pp[0];
-                acc = acc + (double)vpre[u].y * (double)pp[1];
-                acc = acc + (double)vpre[u].z * (double)pp[2];
-                acc = acc + (double)vpre[u].w * (double)pp[3];
-                n += 4;
-            }
-        }
-        // 16 keys (four 16-byte loads) in flight per step
-        for (; n + 16 <= rb; n += 16) {
-            float4 v4[4];
+            const int s = s0 + u;
+            if (s >= steps) break;
+            const f32x4 v = vpre[u];
+            vpre[u] = load_v(min(s + PV, steps - 1));
+            const f32x4 p = *(const f32x4 *)(sc + 32 * s + vk);
+            const int n = k0 + 32 * s + vk;
 #pragma unroll
-            for (int u = 0; u < 4; u++) v4[u] = *(const float4 *)(vr + n + 4 * u);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float * pp = sc + (n + 4 * u - kr.lo);
-                acc = acc + (double)v4[u].x * (double)pp[0];
-                acc = acc + (double)v4[u].y * (double)pp[1];
-                acc = acc + (double)v4[u].z * (double)pp[2];
-                acc = acc + (double)v4[u].w * (double)pp[3];
-            }
+            for (int c = 0; c < 4; c++)
+                o = fma((double)(n + c >= kr.lo && n + c <= kr.hi ? v[c] : 0.0f), (double)(p[c] * inv), o);
         }
-        for (; n + 4 <= rb; n += 4) {
-            const float4 v4 = *(const float4 *)(vr + n);
-            const float * pp = sc + (n - kr.lo);
-            acc = acc + (double)v4.x * (double)pp[0];
-            acc = acc + (double)v4.y * (double)pp[1];
-            acc = acc + (double)v4.z * (double)pp[2];
-            acc = acc + (double)v4.w * (double)pp[3];
-        }
-        for (; n < rb; n++) acc = acc + (double)vr[n] * (double)sc[n - kr.lo];
-        part[pt][d] = acc;
     }
-    __syncthreads();
-    if (tid < HD) {
-        double acc = part[0][tid];
-#pragma unroll
-        for (int pt = 1; pt < PARTS; pt++) acc += part[pt][tid];
-        out[(int64_t)row * H * HD + (int64_t)h * HD + tid] = (float)acc;
-    }
+    o = dpp_sum<0x141>(dpp_sum<0x4E>(dpp_sum<0xB1>(o)));         // the dimension's eight lanes
+    if ((lane & 7) == 0) out[((int64_t)row * H + h) * HD + vd] = (float)o;
 }
 
 extern "C" int dfx_rope_store(const float * qkv, const int32_t * pos, int64_t M, int H, int Hkv, int hd,
@@ -949,60 +919,68 @@ static size_t attn_lds_limit() {
     return v;
 }
 
-// Score-row stride of the matrix-core kernel: whole 16-key tiles, plus 4 floats so
-// rows of a 16-row fragment start in different LDS banks.
-static inline int attn_sstride(int64_t n_keys) { return (int)(((n_keys + 15) / 16) * 16 + 4); }
-
 // Score-row stride of the split-bf16 kernel: whole 32-key tiles, plus 4 floats.
 static inline int attn_split_sstride(int64_t n_keys) { return (int)(((n_keys + 31) / 32) * 32 + 4); }
 
-#ifndef ATTN_NW
-#define ATTN_NW 8   // waves per workgroup of the 128-wide exact kernel
-#endif
-
-// The exact (f64-summed) kernels: scores kept in LDS when a 16-row tile of them fits,
-// else recomputed in three passes.  q_pos0 / window: the causal mask (q_pos0 < 0: none).
+// The exact (f64-summed) kernels; q_pos0 / window: the causal mask (q_pos0 < 0: none).
 static int attn_exact(const float * q, const float * kc, const float * vt, int64_t v_ld, int M, int n_keys, int H,
                       int Hkv, int hd, int q_pos0, int window, float * out, hipStream_t st) {
-    if (M <= 4 && n_keys <= ROWS_MAX_KEYS) {
-        // decoding: one workgroup per (row, head) instead of a 16-row tile per head
+    if ((int64_t)M * H <= attn_cu_count() && n_keys <= ROWS_MAX_KEYS) {
+        // one workgroup per (row, head) where that is one round of the CUs: 8 rows of 28 heads take
+        // 8.1 us over 192 keys and 78 over 4096, as 16-row tiles 13.0 and 165; 16 rows (two rounds)
+        // 14.7 and 152, as tiles 13.1 and 166
         const dim3 grid((unsigned)(M * H));
+        const size_t lds = ((size_t)n_keys + 64) * sizeof(float);
         if (hd == 128)
-            hipLaunchKernelGGL((k_attn_rows<128>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_pos0,
-                               window, out);
+            hipLaunchKernelGGL((k_attn_rows<128>), grid, dim3(1024), lds, st, q, kc, vt, v_ld, M, n_keys, H, Hkv,
+                               q_pos0, window, out);
         else
-            hipLaunchKernelGGL((k_attn_rows<64>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_pos0,
-                               window, out);
+            hipLaunchKernelGGL((k_attn_rows<64>), grid, dim3(512), lds, st, q, kc, vt, v_ld, M, n_keys, H, Hkv,
+                               q_pos0, window, out);
         DFX_CHECK_LAUNCH("dfx_attention (few rows)");
         return DFX_OK;
     }
-    const int sstride = attn_sstride(n_keys);
-    const size_t lds = (size_t)16 * sstride * sizeof(float);
     const int q_tiles = (M + 15) / 16;
-    const dim3 grid((unsigned)(8 * ((H + 7) / 8) * q_tiles));
-    // value columns split over two workgroups per query tile where twice the grid still gives
-    // each CU at most one workgroup (LLaDA-8B at 50 rows, Dream-7B at 12-64 rows: 11-12 % less
-    // attention time; slower on larger grids, where the second workgroup shares a CU)
-    const int vs = 2 * (int)grid.x <= attn_cu_count() ? 2 : 1;
-    const dim3 grid_vs((unsigned)(8 * ((H + 7) / 8) * q_tiles * vs));
-    if (lds <= attn_lds_limit()) {
-        // 128 dims: eight waves, a one-slot key ring (at most 128 VGPRs: four waves per SIMD);
-        // 64 dims: four waves, three slots
-        if (hd == 128 && ATTN_NW == 8)
-            hipLaunchKernelGGL((k_attn_mfma<128, 1, 8>), grid_vs, dim3(512), lds, st, q, kc, vt, v_ld, M, n_keys, H, Hkv,
-                               sstride, q_tiles, q_pos0, window, out, vs);
-        else if (hd == 128)
-            hipLaunchKernelGGL((k_attn_mfma<128, 2, 4>), grid_vs, dim3(256), lds, st, q, kc, vt, v_ld, M, n_keys, H, Hkv,
-                               sstride, q_tiles, q_pos0, window, out, vs);
+    // 16-key tiles that one query tile's rows can see, and per wave of the kernel that keeps scores
+    const int64_t span = q_pos0 >= 0 && window > 0 ? std::min<int64_t>(n_keys, (int64_t)window + 30) : n_keys;
+    const int64_t nt = ((span + 15) / 16 + (span < n_keys) + 7) / 8;
+    if (nt <= 32) {
+        const int units = H * q_tiles;
+        const dim3 g((unsigned)(8 * ((units + 7) / 8)));
+        // Four waves per SIMD (two workgroups per CU, 128 VGPRs) where the units give a CU more
+        // than one workgroup and the scores leave room (128 dims: 6 tiles per wave): 32 heads,
+        // 288 rows over 288 keys 45.7 us against 49.5 with two waves, 768 over 768 191.7 / 204.0;
+        // one workgroup per CU is faster without the register limit (128 over 512: 25.7 / 27.3).
+        const bool two = units > attn_cu_count();
+#define KEEP(HD, NT, WPE)                                                                                             \
+    hipLaunchKernelGGL((k_attn_keep<HD, NT, WPE>), g, dim3(512), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,   \
+                       q_pos0, window, out)
+        if (hd == 128) {
+            if (two && nt <= 2) KEEP(128, 2, 4);
+            else if (two && nt <= 3) KEEP(128, 3, 4);
+            else if (two && nt <= 4) KEEP(128, 4, 4);
+            else if (two && nt <= 6) KEEP(128, 6, 4);
+            else if (nt <= 4) KEEP(128, 4, 2);
+            else if (nt <= 8) KEEP(128, 8, 2);
+            else if (nt <= 16) KEEP(128, 16, 2);
+            else KEEP(128, 32, 2);
+        } else {
+            if (two && nt <= 4) KEEP(64, 4, 4);
+            else if (two && nt <= 8) KEEP(64, 8, 4);
+            else if (nt <= 4) KEEP(64, 4, 2);
+            else if (nt <= 8) KEEP(64, 8, 2);
+            else if (nt <= 16) KEEP(64, 16, 2);
+            else KEEP(64, 32, 2);
+        }
+#undef KEEP
+    } else {   // more scores than the registers hold: recomputed in three passes
+        const dim3 grid((unsigned)(8 * ((H + 7) / 8) * q_tiles));
+        if (hd == 128)
+            hipLaunchKernelGGL((k_attn_long<128>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,
+                               q_pos0, window, out);
         else
-            hipLaunchKernelGGL((k_attn_mfma<64, 3, 4>), grid_vs, dim3(256), lds, st, q, kc, vt, v_ld, M, n_keys, H, Hkv,
-                               sstride, q_tiles, q_pos0, window, out, vs);
-    } else if (hd == 128) {   // score rows longer than the LDS holds: recomputed in three passes
-        hipLaunchKernelGGL((k_attn_long<128>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,
-                           q_pos0, window, out);
-    } else {
-        hipLaunchKernelGGL((k_attn_long<64>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,
-                           q_pos0, window, out);
+            hipLaunchKernelGGL((k_attn_long<64>), grid, dim3(256), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,
+                               q_pos0, window, out);
     }
     DFX_CHECK_LAUNCH("dfx_attention");
     return DFX_OK;

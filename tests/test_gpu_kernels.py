@@ -543,6 +543,41 @@ def test_attention_exact_matches_oracle_and_f64(gpu, M, n_keys, H, Hkv, hd):
     assert np.array_equal(ob.download(np.float32, shape=(M, H, hd)), got)
 
 
+# Edges of the forms behind dfx_attention_causal: one workgroup per row and head up to as many as
+# CUs (8 rows of 32 heads), then 16-row tiles with 2, 3, 4, 6, 8, 16 or 32 key tiles per wave, one
+# or two workgroups per CU, then the recomputing form above 4096 visible keys.
+@pytest.mark.parametrize("M,n_keys,H,Hkv,hd,window", [
+    (8, 33, 32, 4, 128, 0), (9, 33, 32, 4, 128, 0), (1, 1, 3, 1, 128, 0), (2, 1025, 5, 5, 64, 0),
+    (3, 4100, 2, 2, 128, 70), (5, 300, 4, 2, 64, 29),
+    (150, 256, 28, 4, 128, 0), (150, 257, 28, 4, 128, 0), (150, 385, 28, 4, 128, 0), (150, 513, 28, 4, 128, 0),
+    (150, 769, 28, 4, 128, 0), (270, 513, 17, 17, 64, 0), (270, 1025, 17, 17, 64, 0), (270, 1030, 17, 17, 64, 100),
+    (130, 512, 2, 1, 128, 0), (130, 513, 2, 1, 128, 0), (130, 1025, 2, 1, 128, 0), (130, 2049, 2, 1, 128, 0),
+    (130, 4096, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 200), (130, 520, 2, 1, 64, 16),
+    (130, 1030, 2, 2, 64, 0), (130, 2060, 2, 2, 64, 0)])
+def test_attention_causal_matches_f64(gpu, M, n_keys, H, Hkv, hd, window):
+    """Against float64 with the mask.  Scores, probabilities and outputs are rounded to f32 once each
+    (scores of up to about 40 in size move their exponentials by 40 * 2^-24): 4e-6 of the result.
+    Values and keys past the sequence are NaN and must not be read into a result."""
+    q = rng.standard_normal((M, H, hd)).astype(np.float32)
+    v_ld = (n_keys + 15) // 16 * 16 + 16
+    k = np.full((v_ld, Hkv, hd), np.nan, np.float32)
+    k[:n_keys] = rng.standard_normal((n_keys, Hkv, hd))
+    vt = np.full((Hkv, hd, v_ld), np.nan, np.float32)
+    vt[:, :, :n_keys] = rng.standard_normal((Hkv, hd, n_keys))
+    qb, kb, vb, ob = dfx.Buf.of(q), dfx.Buf.of(k), dfx.Buf.of(vt), dfx.Buf(M * H * hd * 4)
+    dfx.check(L().dfx_attention_causal(qb.ptr, kb.ptr, vb.ptr, v_ld, M, n_keys, H, Hkv, hd, n_keys - M, window, ob.ptr,
+                                       None), "attention")
+    got = ob.download(np.float32, shape=(M, H, hd))
+    pos, key = np.arange(n_keys - M, n_keys)[:, None], np.arange(n_keys)[None, :]
+    hide = (key > pos) | ((key <= pos - window) if window else False)
+    for h in range(H):
+        s = q[:, h].astype(np.float64) @ k[:n_keys, h // (H // Hkv)].astype(np.float64).T / np.sqrt(hd)
+        s[hide] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        ref = (p / p.sum(1, keepdims=True)) @ vt[h // (H // Hkv), :, :n_keys].astype(np.float64).T
+        assert rel_l2(got[:, h], ref) < 4e-6, h
+
+
 @pytest.mark.parametrize("M,n_keys,H,Hkv,hd", ATTN_SHAPES)
 def test_attention_split_bf16_matches_f64(gpu, M, n_keys, H, Hkv, hd):
     """The optional DFX_ATTN_SPLIT_BF16: f32 operands split into bf16 hi + mid + lo,
