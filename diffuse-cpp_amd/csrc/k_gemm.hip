@@ -21,7 +21,7 @@
 // rounding difference into whole quantisation steps that grow over the layers;
 // exactness here is what keeps the logits on the CPU path's trajectory.
 //
-// F16 weights run k_gemm_f16: f16 x f16 products (exact) accumulated by MFMA in
+// F16 weights run k_gemm_f16, and k_gemm_f16_w where more rows fill its wider tiles: f16 x f16 products (exact) accumulated by MFMA in
 // f32 (GGML accumulates them in f32/f64 SIMD lanes in its own order).
 //
 // Tiling: workgroup = 4 waves splitting 128 weight rows (32 each); TM tiles of
@@ -1781,6 +1781,166 @@ k_gemm_f16(const uint8_t * __restrict__ W, int N, int K, const half_t * __restri
                       lane, epi);
 }
 
+// F16 GEMM over many rows: WM x WN waves of TM x TN tiles of 32 x 32 (six to nine tiles a wave, so
+// that 5-6 operand reads from LDS feed 6-9 MFMAs where k_gemm_f16's waves read the whole activation
+// tile for four).
+//
+// Both operands go global -> LDS by `buffer_load ... lds`, 32 K elements per step, into a ring of
+// four slots: three steps are in flight, as one CU's misses take 1-2 us and its MFMAs only 0.5 us a
+// step.  A copy moves 16 rows of 64 bytes, lane i fetching chunk (i % 4) ^ f of row i / 4, so that
+// row r keeps its chunk c at slot c ^ f(r) and the rows that a read touches lie in different banks,
+// f(r) = (r >> 1 ^ (r >> 3 & 1)) & 3.  Operands are read one 16-element slice ahead; the barrier stands before
+// the second slice of a step, whose operands are in registers by then, and the copies are spread
+// between the MFMAs (issued together, they kept the matrix cores idle while the waves queued).
+//
+// What bounds it: from cache the loop runs at the matrix cores' rate (0.52 us a step of the 192 x 384
+// tile, 0.48 us of MFMAs at 2.4 GHz); with weights from HBM at 0.84 us, a CU's outstanding misses
+// (about 64 KB) over their latency, which more copies ahead, or lines fetched into L2 ahead of the
+// copies, do not change (10 % slower).  LLaDA-8B at 768 rows, cold weights, us a call, before -> after:
+// gate|up 244 -> 154, down 129 -> 97, Q|K|V 141 -> 92, O 53 -> 48; the whole FFN block 386 -> 274.
+template <int WM, int WN, int TM, int TN>
+__global__ void __launch_bounds__(64 * WM * WN, 2)
+k_gemm_f16_w(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ A, int M,
+             const float * __restrict__ bias, const float * res, float * Y, int64_t ldy,
+             const int32_t * __restrict__ ymap, int n_tiles, int m_tiles, float * __restrict__ ws, int kt_per_split,
+             dfx_epi epi) {
+    constexpr int NW = WM * WN, BM = 32 * WM * TM, BN = 32 * WN * TN;
+    constexpr int CA = BM / 16, C = (BM + BN) / 16, CW = (C + NW - 1) / NW, CMIN = C / NW;   // copies: A, all, per wave
+    constexpr int SH = (BM + BN) * 32;   // halves per slot
+    constexpr int NM = TM * TN, G = 3;   // MFMAs and issue groups per slice
+    static_assert(CW <= 6 && TM <= 4 && TN <= 4, "copies");
+    __shared__ __attribute__((aligned(1024))) half_t S0[SH], S1[SH], S2[SH], S3[SH];
+    auto slot = [&](auto stage) __attribute__((always_inline)) -> half_t * {
+        constexpr int s = decltype(stage)::value & 3;
+        if constexpr (s == 0) return S0;
+        else if constexpr (s == 1) return S1;
+        else if constexpr (s == 2) return S2;
+        else return S3;
+    };
+    const int per_pass = 8 * ((n_tiles + 7) / 8) * m_tiles;
+    const int z = blockIdx.x / per_pass, L = blockIdx.x - z * per_pass, xcd = L & 7, jj = L >> 3;
+    const int ty = jj % m_tiles, tx = 8 * (jj / m_tiles) + xcd;
+    if (tx >= n_tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, l32 = lane & 31;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wv / WN, wn = wv % WN;
+    const int n0 = tx * BN, m0 = ty * BM;
+    const int n_kt = K / 32;
+    const int kt0 = z * kt_per_split, kt1 = min(kt0 + kt_per_split, n_kt);
+    const int64_t row_bytes = (int64_t)K * 2;
+    const uint8_t * const At = A + m0 * row_bytes, * const Wt = W + n0 * row_bytes;
+    uint32_t off[8];
+#pragma unroll
+    for (int j = 0; j < CW; j++) {
+        const int c = min(wv + NW * j, C - 1);
+        const int r16 = lane >> 2;
+        const int row = c < CA ? min(16 * c + r16, M - 1 - m0) : min(16 * (c - CA) + r16, N - 1 - n0);
+        off[j] = (uint32_t)row * (uint32_t)row_bytes + ((((lane & 3) ^ (r16 >> 1) ^ (r16 >> 3)) & 3) << 4);
+    }
+    auto copy = [&](auto stage, auto jc, int kt_req) __attribute__((always_inline)) {
+        constexpr int j = decltype(jc)::value;
+        if constexpr (j < CW) {
+            const int c = wv + NW * j;
+            if (NW * j + NW <= C || c < C) {
+                const __amdgpu_buffer_rsrc_t r =
+                    __builtin_amdgcn_make_buffer_rsrc((void *)(c < CA ? At : Wt), 0, 0xFFFFFFFF, 0x00020000);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)(slot(stage) + c * 512), 16, off[j],
+                                                         min(kt_req, n_kt - 1) * 64, 0, 0);
+            }
+        }
+    };
+    auto issue = [&](auto stage, int kt_req) __attribute__((always_inline)) {
+        copy(stage, std::integral_constant<int, 0>{}, kt_req);
+        copy(stage, std::integral_constant<int, 1>{}, kt_req);
+        copy(stage, std::integral_constant<int, 2>{}, kt_req);
+        copy(stage, std::integral_constant<int, 3>{}, kt_req);
+        copy(stage, std::integral_constant<int, 4>{}, kt_req);
+        copy(stage, std::integral_constant<int, 5>{}, kt_req);
+    };
+    struct frag { half8 a[4], b[4]; } F[2];
+    const int f = ((l32 >> 1) ^ (l32 >> 3 & 1)) & 3;
+    // operand x of the slice's TM + TN (A first)
+    auto load1 = [&](auto stage, auto slice, frag & d, int x) __attribute__((always_inline)) {
+        constexpr int t = decltype(slice)::value;
+        const half_t * s = slot(stage) + ((2 * t + hl) ^ f) * 8;
+        if (x < TM) d.a[x] = *(const half8 *)(s + ((wm * TM + x) * 32 + l32) * 32);
+        else d.b[x - TM] = *(const half8 *)(s + BM * 32 + ((wn * TN + x - TM) * 32 + l32) * 32);
+    };
+    struct accs { float16v t[16]; } acc;
+#pragma unroll
+    for (int i = 0; i < NM; i++) acc.t[i] = float16v{};
+    auto group = [&](auto stage_l, auto slice_l, frag & nxt, const frag & cur, auto stage_c, auto cj, int kt_c,
+                     auto gc) __attribute__((always_inline)) {
+        constexpr int g = decltype(gc)::value, X = TM + TN;
+#pragma unroll
+        for (int x = g * X / G; x < (g + 1) * X / G; x++) load1(stage_l, slice_l, nxt, x);
+        copy(stage_c, cj, kt_c);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = g * NM / G; i < (g + 1) * NM / G; i++)
+            acc.t[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.a[i / TN], cur.b[i % TN], acc.t[i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using std::integral_constant;
+    auto step = [&](auto stage, int kt) __attribute__((always_inline)) {
+        constexpr int s = decltype(stage)::value;
+        constexpr integral_constant<int, (s + 1) & 3> s1{};
+        constexpr integral_constant<int, (s + 3) & 3> s3{};
+        constexpr integral_constant<int, 0> i0{};
+        constexpr integral_constant<int, 1> i1{};
+        constexpr integral_constant<int, 2> i2{};
+        group(stage, i1, F[1], F[0], s3, i0, kt + 3, i0);
+        group(stage, i1, F[1], F[0], s3, i1, kt + 3, i1);
+        group(stage, i1, F[1], F[0], s3, i2, kt + 3, i2);
+        constexpr int SOFAR = CMIN < 3 ? CMIN : 3;
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm(CMIN + SOFAR, 0));
+        barrier_only();
+        __builtin_amdgcn_sched_barrier(0);
+        group(s1, i0, F[0], F[1], s3, integral_constant<int, 3>{}, kt + 3, i0);
+        group(s1, i0, F[0], F[1], s3, integral_constant<int, 4>{}, kt + 3, i1);
+        group(s1, i0, F[0], F[1], s3, integral_constant<int, 5>{}, kt + 3, i2);
+    };
+    issue(integral_constant<int, 0>{}, kt0);
+    issue(integral_constant<int, 1>{}, kt0 + 1);
+    issue(integral_constant<int, 2>{}, kt0 + 2);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm(2 * CMIN, 0));
+    barrier_only();
+#pragma unroll
+    for (int x = 0; x < TM + TN; x++) load1(integral_constant<int, 0>{}, integral_constant<int, 0>{}, F[0], x);
+    for (int kt = kt0; kt < kt1; kt += 4) {
+        step(integral_constant<int, 0>{}, kt);
+        step(integral_constant<int, 1>{}, kt + 1);
+        step(integral_constant<int, 2>{}, kt + 2);
+        step(integral_constant<int, 3>{}, kt + 3);
+    }
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm(0, 0));
+    // one copy of the epilogue's code, the tile picked by uniform branches (an indexed read of the
+    // accumulators would select among all of them)
+    auto tile = [&](auto ic, int i, float16v & v) __attribute__((always_inline)) {
+        constexpr int t = decltype(ic)::value;
+        if constexpr (t < NM)
+            if (i == t) {
+                v = acc.t[t];
+                asm volatile("" : "+v"(v));
+            }
+    };
+#pragma clang loop unroll(disable)
+    for (int i = 0; i < NM; i++) {
+        float16v v;
+        tile(integral_constant<int, 0>{}, i, v);
+        tile(integral_constant<int, 1>{}, i, v);
+        tile(integral_constant<int, 2>{}, i, v);
+        tile(integral_constant<int, 3>{}, i, v);
+        tile(integral_constant<int, 4>{}, i, v);
+        tile(integral_constant<int, 5>{}, i, v);
+        tile(integral_constant<int, 6>{}, i, v);
+        tile(integral_constant<int, 7>{}, i, v);
+        tile(integral_constant<int, 8>{}, i, v);
+        epilogue_tile(v, m0 + (wm * TM + i / TN) * 32, n0 + (wn * TN + i % TN) * 32 + l32, M, N, bias, res, Y, ldy, ymap,
+                      ws, z, lane, epi);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // F32 weights (GGML's vec_dot_type of F32 is F32: activations are not converted)
 // ---------------------------------------------------------------------------
@@ -2097,6 +2257,58 @@ static int launch_f16(const void * w, int N, int K, const void * act, int M, con
     DFX_CHECK_LAUNCH("dfx_gemm f16");
     if (S > 1) return reduce_or_defer(ws, S, M, N, bias, res, y, ldy, ymap, st, defer, epi);
     return DFX_OK;
+}
+
+template <int WM, int WN, int TM, int TN>
+static int launch_f16_w(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
+                        float * y, int64_t ldy, const int32_t * ymap, void * ws, int S, hipStream_t st, int * defer,
+                        dfx_epi epi) {
+    constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+    const int n_tiles = (N + BN - 1) / BN, m_tiles = (M + BM - 1) / BM;
+    // K steps per slice: a multiple of 8 (K is one of 256 elements)
+    const int n_kt = K / 32, per = (n_kt + 8 * S - 1) / (8 * S) * 8;
+    S = (n_kt + per - 1) / per;
+    const int per_pass = 8 * ((n_tiles + 7) / 8) * m_tiles;
+    hipLaunchKernelGGL((k_gemm_f16_w<WM, WN, TM, TN>), dim3((unsigned)(per_pass * S)), dim3(64 * WM * WN), 0, st,
+                       (const uint8_t *)w, N, K, (const uint8_t *)act, M, bias, res, y, ldy, ymap, n_tiles, m_tiles,
+                       S > 1 ? (float *)ws : nullptr, per, epi);
+    DFX_CHECK_LAUNCH("dfx_gemm f16");
+    if (S > 1) return reduce_or_defer(ws, S, M, N, bias, res, y, ldy, ymap, st, defer, epi);
+    return DFX_OK;
+}
+
+// Tiles and K slices of an F16 GEMM over more than 256 rows, by the time that each choice would
+// take: rounds over the CUs (one workgroup each) x K steps of 32 x the tile's measured time a step
+// with cold weights, and for split K the slices' traffic at 4 TB/s and the reduction's launch.
+// k_gemm_f16's own tiles (128 x 128, two workgroups per CU) are among the choices: at 512 rows of
+// N = 12288 they take 82 us against 88 (192 x 256).  Up to 256 rows they are the better ones at
+// most shapes (N = 24576: 93 us against 109 at 256 rows, 67 against 76 at 128).
+enum f16_tiles { F16_128x128, F16_192x128, F16_192x256, F16_256x256, F16_192x384 };
+struct f16_choice {
+    f16_tiles tiles;
+    int S;
+};
+static f16_choice f16_choose(int64_t M, int64_t N, int64_t K, size_t ws_bytes) {
+    static const struct { f16_tiles tiles; int bm, bn, max_s; double us; } form[] = {
+        {F16_192x128, 192, 128, 4, 0.47}, {F16_192x256, 192, 256, 4, 0.72},
+        {F16_256x256, 256, 256, 1, 0.85}, {F16_192x384, 192, 384, 1, 1.05}};
+    const double steps = (double)K / 32;
+    auto slices_us = [&](int S) { return S > 1 ? S * 8e-6 * (double)M * (double)N / 4.0 + 3.0 : 0.0; };
+    const int s0 = f16_splits(4, M, N, K, ws_bytes);
+    const double n0 = (double)((N + 127) / 128 * ((M + 127) / 128) * s0);
+    f16_choice best{F16_128x128, s0};
+    double best_us = steps / s0 * (n0 <= 256 ? 0.45 : n0 <= 512 ? 0.68 : 0.68 * 1.15 * n0 / 512) + slices_us(s0);
+    if (M <= 256) return best;
+    for (const auto & f : form)
+        for (int S = 1; S <= f.max_s && (S == 1 || (size_t)S * M * N * sizeof(float) <= ws_bytes); S *= 2) {
+            const int64_t n = (N + f.bn - 1) / f.bn * ((M + f.bm - 1) / f.bm) * S;
+            const double us = (double)((n + 255) / 256) * steps / S * f.us + slices_us(S);
+            if (us < best_us) {
+                best_us = us;
+                best = {f.tiles, S};
+            }
+        }
+    return best;
 }
 
 template <int TM>
@@ -2855,6 +3067,13 @@ int dfx_gemm_ex(int wtype, const void * w, int64_t N, int64_t K, const void * ac
         case DFX_TYPE_Q6_K: return dispatch_q6k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
         case DFX_TYPE_Q8_0: return dispatch_mmq<DFX_TYPE_Q8_0>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
         case DFX_TYPE_F16:
+            switch (f16_choice c = f16_choose(m, n, k, ws ? ws_bytes : 0); c.tiles) {
+                case F16_192x128: return launch_f16_w<2, 2, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
+                case F16_192x256: return launch_f16_w<2, 4, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
+                case F16_256x256: return launch_f16_w<2, 4, 4, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
+                case F16_192x384: return launch_f16_w<2, 4, 3, 3>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
+                case F16_128x128: break;
+            }
             switch (pick_tm(m, 4)) {
                 case 1: return launch_f16<1>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
                 case 2: return launch_f16<2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
