@@ -2738,22 +2738,22 @@ static int dispatch_mmq(const void * w, int N, int K, const void * act, int M, c
 // ---------------------------------------------------------------------------
 // Q4_K / Q6_K matrix-vector kernels: at most DFX_GEMV_M activation rows (decoding)
 // ---------------------------------------------------------------------------
-// One wave per pair of output columns (n, n + 16) and pass set, n = 32 (p / 16) + p % 16 for
-// pair p: the pairs the SwiGLU and RoPE epilogues combine.  A pass is 16 super-blocks (two
-// chunks of 2048); lane l takes the 64-element group l % 4 of super-block l / 4 of each
-// pass, for both columns and all rows.  Rows of one pass: four pairs per workgroup, a wave
-// each.  Longer rows (SPLIT, e.g. the FFN down projection): a workgroup per pair with one
-// wave per pass (up to 16, each taking every ws-th pass beyond that), so every pass's weight
-// loads are in flight at once.  Integer dot products come from v_dot4_i32_i8 on the
-// natural-order int8 activation plane (nibbles and 6-bit quants are non-negative bytes),
-// exactly, in int32; the four lanes of a super-block add them (DPP quad permutes), and every
-// lane then runs the exact float order over the super-blocks of each chunk (x and d_a read
-// from the lanes that hold them): x = d_w*isum (Q4_K: x = fma(-dmin_w, msum, x));
-// S = fma(d_a, x, S).  The chunk sums are added in chunk order, T = T + S, in the wave or,
-// after a barrier, from LDS by the pair's first wave.  No MFMA: at these row counts the
-// weights' HBM stream sets the time.
-constexpr int GEMV_MAX_CHUNKS = 64;     // K <= 131072 for the pass-split form
-
+// Two workgroups per CU stream the weights: each owns a contiguous range of column pairs
+// (n, n + 16), n = 32 (p / 16) + p % 16 for pair p, the pairs that the SwiGLU and RoPE epilogues
+// combine.  Four lanes take one super-block of a pair, lane g the 64-element group g, and the
+// next item's weights are loaded before this one's are used.  The int8 activations and their sums
+// lie in LDS (16-byte pieces plane by plane: consecutive lanes read consecutive pieces).  Integer
+// dot products come from v_dot4_i32_i8 (nibbles and 6-bit quants are non-negative bytes),
+// exactly, in int32; the four lanes of a super-block add them (DPP quad permutes) and
+// x = d_w*isum (Q4_K: x = fma(-dmin_w, msum, x)) goes to LDS.  After one barrier a lane per
+// output runs the exact float order over all super-blocks: S = fma(d_a, x, S) in each chunk of 8,
+// T = T + S.
+//
+// What bounds it: HBM at the widest (5.5 TB/s over the vocab heads), below that the latency of the
+// first loads.  A wave per pair of columns, which this replaces, ran the chains wave-wide from
+// v_readlane and loaded and converted the activations for every pair.  One row, us, before -> after:
+// Dream-7B gate|up 21.0 -> 16.8, down 16.3 -> 13.2, Q4_K head 66.8 -> 55.7, Q6_K head 111 -> 84;
+// LLaDA-8B gate|up 16.0 -> 14.0, down 11.5 -> 10.3.
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }
@@ -2764,11 +2764,6 @@ __device__ __forceinline__ int quad_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);   // quad_perm [1, 0, 3, 2]
     v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);   // quad_perm [2, 3, 0, 1]
     return v;
-}
-
-// the value of a lane known at compile time, as a wave-uniform value
-__device__ __forceinline__ float lane_value(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // One output of the matrix-vector kernels through the epilogue: v = row m at column n,
@@ -2808,205 +2803,222 @@ __device__ __forceinline__ void gemv_store(float v, float w, int m, int n, int N
     Y[o] = v;
 }
 
-template <int WT, int MR, bool SPLIT>
-__global__ void __launch_bounds__(1024) k_gemv(const uint8_t * __restrict__ W, int N, int K,
-                                              const uint8_t * __restrict__ act, int M, const float * __restrict__ bias,
-                                              const float * res, float * Y, int64_t ldy,
-                                              const int32_t * __restrict__ ymap, dfx_epi epi) {
+// Threads of a workgroup, two of which share a CU: 8 waves each leave 128 registers a lane, which
+// Q6_K over several rows overflows (the head at four rows 140 us with the spills, 118 with 6 waves).
+constexpr int gemv_threads(int wt, int rows) { return wt == DFX_TYPE_Q6_K && rows > 1 ? 384 : 512; }
+
+// Raw weights of one item: a lane's share of a super-block of two columns.
+template <int WT> struct gemv_raw;
+template <> struct gemv_raw<DFX_TYPE_Q4_K> { u32x4 h[2], q[2][2]; };
+template <> struct gemv_raw<DFX_TYPE_Q6_K> { u32x4 la[2], lb[2], qh[2], sc[2]; uint32_t d[2]; };
+
+template <int WT, int MR, bool ONE>
+__global__ void __launch_bounds__(gemv_threads(WT, MR)) __attribute__((amdgpu_waves_per_eu(gemv_threads(WT, MR) / 128)))
+k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
+       const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
+       dfx_epi epi) {
 #pragma clang fp contract(off)
     constexpr bool Q4 = WT == DFX_TYPE_Q4_K;
     constexpr int SB = Q4 ? SB_Q4_K : SB_Q6_K;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int ws = SPLIT ? (int)(blockDim.x >> 6) : 1;   // waves per pair
-    const int p = SPLIT ? (int)blockIdx.x : (int)blockIdx.x * 4 + wv, part = SPLIT ? wv : 0;
-    const bool pair_live = p < N / 2;                    // the whole wave
-    if (!SPLIT && !pair_live) return;
-    const int ncol[2] = {32 * (p >> 4) + (p & 15), 32 * (p >> 4) + (p & 15) + 16};
-    const int nsb = K >> 8, g = lane & 3, sbl = lane >> 2;
+    extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
+    const int tid = threadIdx.x, g = tid & 3;
+    const int nsb = K >> 8, T4 = (int)blockDim.x >> 2;   // items per pass
+    const int p0 = (int)((int64_t)blockIdx.x * (N / 2) / gridDim.x);
+    const int ncol = 2 * ((int)((int64_t)(blockIdx.x + 1) * (N / 2) / gridDim.x) - p0);
+    const int items = nsb * (ncol / 2);
+    const int a_bytes = ONE ? 0 : MR * K, b_bytes = ONE ? 0 : MR * nsb * 32;
+    u32x4 * as = (u32x4 *)gemv_lds;                           // [MR][4][nsb * 4]: piece i of group g
+    uint2 * bs = (uint2 *)(gemv_lds + a_bytes);               // [MR][nsb * 4]: the group's sums
+    float * xs = (float *)(gemv_lds + a_bytes + b_bytes);     // [MR][nsb][ncol]
+    float * ds = xs + MR * nsb * ncol;                        // [MR][nsb]
     const act_layout Lay = act_layout_of(Q4 ? CONV_Q8_K_P4 : CONV_Q8_K_P6, M, K);
-    const int8_t * a8 = (const int8_t *)(act + Lay.i8);
-    const float * ad = (const float *)(act + Lay.d);     // [nsb][mq]
-    const uint16_t * abs = (const uint16_t *)(act + Lay.bs);   // [M][K/16], exact small integers
+    const float * ad = (const float *)(act + Lay.d);                 // [nsb][mq]
+    const uint16_t * abs = (const uint16_t *)(act + Lay.bs);         // [M][K/16], exact small integers
     const int64_t rb = (int64_t)nsb * SB;
-    [[maybe_unused]] __shared__ float sS[SPLIT ? GEMV_MAX_CHUNKS * 2 * MR : 1];
-    float T[2][MR];
-#pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int m = 0; m < MR; m++) T[c][m] = 0.0f;
-
-    for (int sb0 = 16 * part; pair_live && sb0 < nsb; sb0 += 16 * ws) {
-        const int sbc = min(sb0 + sbl, nsb - 1);          // clamped: lanes past the end add nothing
-        const bool live = sb0 + sbl < nsb;
-        float x[2][MR];
+    auto column = [&](int c) __attribute__((always_inline)) -> int {
+        const int p = p0 + (c >> 1);
+        return 32 * (p >> 4) + (p & 15) + 16 * (c & 1);
+    };
+    // 16 bytes of row m: piece i of group gg of super-block sb; and the sums that go with the group
+    auto piece = [&](int m, int sb, int gg, int i) __attribute__((always_inline)) -> u32x4 {
+        const int8_t * row = (const int8_t *)(act + Lay.i8) + (int64_t)min(m, M - 1) * K + sb * 256;
+        return *(const u32x4 *)(row + (Q4 ? 64 * gg + 16 * i : 128 * (gg >> 1) + 32 * i + 16 * (gg & 1)));
+    };
+    auto sums = [&](int m, int sb, int gg) __attribute__((always_inline)) -> uint2 {
+        const uint16_t * row = abs + (int64_t)min(m, M - 1) * (K / 16) + sb * 16;
+        auto sum = [&](int i) __attribute__((always_inline)) -> int { return (int)h2f(row[i]); };
+        if constexpr (Q4)   // of the two sub-blocks
+            return make_uint2((uint32_t)(sum(4 * gg) + sum(4 * gg + 1)), (uint32_t)(sum(4 * gg + 2) + sum(4 * gg + 3)));
+        // of the four strips, 16 bits each
+        const int e = 8 * (gg >> 1) + (gg & 1);
+        return make_uint2(((uint32_t)sum(e) & 0xFFFFu) | ((uint32_t)sum(e + 2) << 16),
+                          ((uint32_t)sum(e + 4) & 0xFFFFu) | ((uint32_t)sum(e + 6) << 16));
+    };
+    // item t: pair t / nsb of the workgroup, super-block t % nsb (past the end: the last again)
+    auto load = [&](int t_req, gemv_raw<WT> & r) __attribute__((always_inline)) {
+        const int t = min(t_req, items - 1), pl = t / nsb, sb = t - pl * nsb;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-            const uint8_t * blk = W + (int64_t)ncol[c] * rb + (int64_t)sbc * SB;
-            int isum[MR], msum[MR];
-            float dw, dmw = 0.0f;
+            const uint8_t * blk = W + (int64_t)column(2 * pl + c) * rb + (int64_t)sb * SB;
             if constexpr (Q4) {
                 // header {d, dmin, scales[12]}, then 32 nibble bytes of group g (sub-blocks 2g, 2g+1)
-                const u32x4 h = *(const u32x4 *)blk;
-                const u32x4 q0 = *(const u32x4 *)(blk + 16 + 32 * g), q1 = *(const u32x4 *)(blk + 32 + 32 * g);
-                const q4k_sm sm = q4k_unpack(h);
-                const uint32_t scw = g < 2 ? sm.sc_lo : sm.sc_hi, mnw = g < 2 ? sm.mn_lo : sm.mn_hi;
-                const int sh = 16 * (g & 1);
-                const int sc0 = (scw >> sh) & 0xFF, sc1 = (scw >> (sh + 8)) & 0xFF;
-                const int mn0 = (mnw >> sh) & 0xFF, mn1 = (mnw >> (sh + 8)) & 0xFF;
-                dw = h2f((uint16_t)(h.x & 0xFFFFu));
-                dmw = h2f((uint16_t)(h.x >> 16));
-                const uint32_t qw[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
-#pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    const int mm = min(m, M - 1);
-                    const int8_t * ar = a8 + (int64_t)mm * K + (int64_t)sbc * 256 + 64 * g;
-                    const u32x4 a0 = *(const u32x4 *)ar, a1 = *(const u32x4 *)(ar + 16);
-                    const u32x4 a2 = *(const u32x4 *)(ar + 32), a3 = *(const u32x4 *)(ar + 48);
-                    const uint32_t aw[16] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w,
-                                             a2.x, a2.y, a2.z, a2.w, a3.x, a3.y, a3.z, a3.w};
-                    int slo = 0, shi = 0;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) {
-                        slo = sdot4(qw[i] & 0x0F0F0F0Fu, aw[i], slo);
-                        shi = sdot4((qw[i] >> 4) & 0x0F0F0F0Fu, aw[8 + i], shi);
-                    }
-                    isum[m] = sc0 * slo + sc1 * shi;
-                    const uint2 bsw = *(const uint2 *)(abs + (int64_t)mm * (K / 16) + sbc * 16 + 4 * g);
-                    const int b0 = (int)h2f((uint16_t)(bsw.x & 0xFFFFu)), b1 = (int)h2f((uint16_t)(bsw.x >> 16));
-                    const int b2 = (int)h2f((uint16_t)(bsw.y & 0xFFFFu)), b3 = (int)h2f((uint16_t)(bsw.y >> 16));
-                    msum[m] = mn0 * (b0 + b1) + mn1 * (b2 + b3);
-                }
+                r.h[c] = *(const u32x4 *)blk;
+                r.q[c][0] = *(const u32x4 *)(blk + 16 + 32 * g);
+                r.q[c][1] = *(const u32x4 *)(blk + 32 + 32 * g);
             } else {
                 // group g: half hf = g / 2, quants l = 16 (g % 2) .. +15 of each of the four
                 // 32-element strips k (elements 128 hf + 32 k + l, sub-block 8 hf + 2 k + g % 2)
                 const int hf = g >> 1, lh = 16 * (g & 1);
-                const u32x4 la = *(const u32x4 *)(blk + 64 * hf + lh), lb = *(const u32x4 *)(blk + 64 * hf + 32 + lh);
-                const u32x4 qh = *(const u32x4 *)(blk + 128 + 32 * hf + lh);
-                const u32x4 scv = *(const u32x4 *)(blk + 192);
-                dw = h2f(*(const uint16_t *)(blk + 208));
-                const uint32_t law[4] = {la.x, la.y, la.z, la.w}, lbw[4] = {lb.x, lb.y, lb.z, lb.w};
-                const uint32_t qhw[4] = {qh.x, qh.y, qh.z, qh.w};
-                uint32_t u[4][4];
-#pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    u[0][t] = (law[t] & 0x0F0F0F0Fu) | ((qhw[t] << 4) & 0x30303030u);
-                    u[1][t] = (lbw[t] & 0x0F0F0F0Fu) | ((qhw[t] << 2) & 0x30303030u);
-                    u[2][t] = ((law[t] >> 4) & 0x0F0F0F0Fu) | (qhw[t] & 0x30303030u);
-                    u[3][t] = ((lbw[t] >> 4) & 0x0F0F0F0Fu) | ((qhw[t] >> 2) & 0x30303030u);
-                }
-                int sck[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int j = 8 * hf + 2 * k + (g & 1);
-                    sck[k] = (int)(int8_t)((scv[j >> 2] >> (8 * (j & 3))) & 0xFFu);
-                }
-#pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    const int mm = min(m, M - 1);
-                    const int8_t * ar = a8 + (int64_t)mm * K + (int64_t)sbc * 256 + 128 * hf + lh;
-                    const uint16_t * br = abs + (int64_t)mm * (K / 16) + sbc * 16 + 8 * hf + (g & 1);
-                    int acc = 0;
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const u32x4 a = *(const u32x4 *)(ar + 32 * k);
-                        int us = 0;
-                        us = sdot4(u[k][0], a.x, us);
-                        us = sdot4(u[k][1], a.y, us);
-                        us = sdot4(u[k][2], a.z, us);
-                        us = sdot4(u[k][3], a.w, us);
-                        const int bsum = (int)h2f(br[2 * k]);
-                        acc += sck[k] * (us - 32 * bsum);
-                    }
-                    isum[m] = acc;
-                    msum[m] = 0;
-                }
+                r.la[c] = *(const u32x4 *)(blk + 64 * hf + lh);
+                r.lb[c] = *(const u32x4 *)(blk + 64 * hf + 32 + lh);
+                r.qh[c] = *(const u32x4 *)(blk + 128 + 32 * hf + lh);
+                r.sc[c] = *(const u32x4 *)(blk + 192);
+                r.d[c] = *(const uint16_t *)(blk + 208);
             }
-            // the super-block's four lanes (consecutive) hold its four groups
+        }
+    };
+    auto compute = [&](int t, const gemv_raw<WT> & r) __attribute__((always_inline)) {
+        const int pl = t / nsb, sb = t - pl * nsb;
 #pragma unroll
-            for (int m = 0; m < MR; m++) {
-                const int is = quad_sum(isum[m]);
+        for (int m = 0; m < MR; m++) {
+            u32x4 a[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                a[i] = ONE ? piece(m, sb, g, i) : as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + g];
+            const uint2 b = ONE ? sums(m, sb, g) : bs[m * nsb * 4 + 4 * sb + g];
+            float x[2];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
                 if constexpr (Q4) {
-                    const int ms = quad_sum(msum[m]);
-                    x[c][m] = fmaf(-dmw, (float)ms, dw * (float)is);
+                    const q4k_sm sm = q4k_unpack(r.h[c]);
+                    const int sh = 16 * (g & 1);
+                    const uint32_t sc = (g < 2 ? sm.sc_lo : sm.sc_hi) >> sh, mn = (g < 2 ? sm.mn_lo : sm.mn_hi) >> sh;
+                    int slo = 0, shi = 0;
+#pragma unroll
+                    for (int i = 0; i < 8; i++) {
+                        const uint32_t w = r.q[c][i >> 2][i & 3];
+                        slo = sdot4(w & 0x0F0F0F0Fu, a[i >> 2][i & 3], slo);
+                        shi = sdot4((w >> 4) & 0x0F0F0F0Fu, a[2 + (i >> 2)][i & 3], shi);
+                    }
+                    const int is = quad_sum((int)(sc & 0xFF) * slo + (int)((sc >> 8) & 0xFF) * shi);
+                    const int ms = quad_sum((int)(mn & 0xFF) * (int)b.x + (int)((mn >> 8) & 0xFF) * (int)b.y);
+                    const float dw = h2f((uint16_t)(r.h[c].x & 0xFFFFu)), dmw = h2f((uint16_t)(r.h[c].x >> 16));
+                    x[c] = fmaf(-dmw, (float)ms, dw * (float)is);
                 } else {
-                    x[c][m] = dw * (float)is;
+                    // scales of the lane's four strips: bytes 8 hf + 2 k + g % 2
+                    const uint32_t s0 = (g >> 1 ? r.sc[c].z : r.sc[c].x) >> (8 * (g & 1));
+                    const uint32_t s1 = (g >> 1 ? r.sc[c].w : r.sc[c].y) >> (8 * (g & 1));
+                    const int sck[4] = {(int)(int8_t)(s0 & 0xFF), (int)(int8_t)((s0 >> 16) & 0xFF),
+                                        (int)(int8_t)(s1 & 0xFF), (int)(int8_t)((s1 >> 16) & 0xFF)};
+                    const int b32[4] = {32 * (int)(int16_t)(b.x & 0xFFFF), 32 * ((int)b.x >> 16),
+                                        32 * (int)(int16_t)(b.y & 0xFFFF), 32 * ((int)b.y >> 16)};
+                    int us[4] = {0, 0, 0, 0}, acc = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t wa = r.la[c][i], wb = r.lb[c][i], wh = r.qh[c][i];
+                        us[0] = sdot4((wa & 0x0F0F0F0Fu) | ((wh << 4) & 0x30303030u), a[0][i], us[0]);
+                        us[1] = sdot4((wb & 0x0F0F0F0Fu) | ((wh << 2) & 0x30303030u), a[1][i], us[1]);
+                        us[2] = sdot4(((wa >> 4) & 0x0F0F0F0Fu) | (wh & 0x30303030u), a[2][i], us[2]);
+                        us[3] = sdot4(((wb >> 4) & 0x0F0F0F0Fu) | ((wh >> 2) & 0x30303030u), a[3][i], us[3]);
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) acc += sck[k] * (us[k] - b32[k]);
+                    x[c] = h2f((uint16_t)r.d[c]) * (float)quad_sum(acc);
                 }
-                if (!live) x[c][m] = 0.0f;
             }
+            if (g == 0) *(float2 *)(xs + ((size_t)m * nsb + sb) * ncol + 2 * pl) = make_float2(x[0], x[1]);
         }
-        // each lane's super-block scale of the activation rows, loaded together for the pass
-        float dam[MR];
-#pragma unroll
-        for (int m = 0; m < MR; m++) dam[m] = ad[(int64_t)sbc * Lay.mq + min(m, M - 1)];
-        // the pass's two chunks of 8 super-blocks: S = fma(d_a, x, S) in order, T = T + S
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int first = sb0 + 8 * h;
-            if (first >= nsb) break;
-            float S[2][MR];
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int m = 0; m < MR; m++) S[c][m] = 0.0f;
-            for (int i = 0; i < 8 && first + i < nsb; i++) {
-#pragma unroll
-                for (int m = 0; m < MR; m++) {
-                    const float da = lane_value(dam[m], 32 * h + 4 * i);
-#pragma unroll
-                    for (int c = 0; c < 2; c++) S[c][m] = fmaf(da, lane_value(x[c][m], 32 * h + 4 * i), S[c][m]);
-                }
-            }
-            if constexpr (!SPLIT) {
-#pragma unroll
-                for (int c = 0; c < 2; c++)
-#pragma unroll
-                    for (int m = 0; m < MR; m++) T[c][m] = T[c][m] + S[c][m];
-            } else if (lane == 0) {
-                float * d = sS + (first >> 3) * 2 * MR;
-#pragma unroll
-                for (int c = 0; c < 2; c++)
-#pragma unroll
-                    for (int m = 0; m < MR; m++) d[c * MR + m] = S[c][m];
-            }
+    };
+    gemv_raw<WT> r0, r1;
+    int t = tid >> 2;
+    load(t, r0);
+    if constexpr (!ONE) {
+        for (int u = tid; u < MR * nsb * 16; u += (int)blockDim.x) {
+            const int m = u / (nsb * 16), v = u - m * nsb * 16, sb = v >> 4, gg = (v >> 2) & 3, i = v & 3;
+            as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + gg] = piece(m, sb, gg, i);
+        }
+        for (int u = tid; u < MR * nsb * 4; u += (int)blockDim.x) {
+            const int m = u / (nsb * 4), v = u - m * nsb * 4;
+            bs[u] = sums(m, v >> 2, v & 3);
         }
     }
-    if constexpr (SPLIT) {
+    for (int u = tid; u < MR * nsb; u += (int)blockDim.x) {
+        const int m = u / nsb, sb = u - m * nsb;
+        ds[u] = ad[(int64_t)sb * Lay.mq + min(m, M - 1)];
+    }
+    // (a quad's four lanes share its items, so quad_sum sees all of them or none)
+    if constexpr (ONE) {
+        if (t < items) compute(t, r0);
+    } else {
         __syncthreads();
-        if (part != 0 || !pair_live) return;
-        const float * d = sS;
-        for (int ch = 0; ch < (nsb + 7) >> 3; ch++)
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int m = 0; m < MR; m++) T[c][m] = T[c][m] + d[ch * 2 * MR + c * MR + m];
+        for (; t < items; t += 2 * T4) {
+            load(t + T4, r1);
+            compute(t, r0);
+            load(t + 2 * T4, r0);
+            if (t + T4 < items) compute(t + T4, r1);
+        }
     }
-    // lane 2m + c stores row m of column c
+    __syncthreads();
+    for (int o = tid; o < MR * ncol; o += (int)blockDim.x) {   // ncol is even: o ^ 1 is the paired column of the same row
+        const int m = o / ncol, c = o - m * ncol;
+        const float * xr = xs + (size_t)m * nsb * ncol + c, * dr = ds + m * nsb;
+        float T = 0.0f;
+        for (int sb0 = 0; sb0 < nsb; sb0 += 8) {
+            float xv[8], dv[8], S = 0.0f;
 #pragma unroll
-    for (int m = 0; m < MR; m++)
+            for (int i = 0; i < 8; i++) {
+                const int sb = min(sb0 + i, nsb - 1);
+                xv[i] = xr[sb * ncol];
+                dv[i] = dr[sb];
+            }
 #pragma unroll
-        for (int c = 0; c < 2; c++)
-            if (lane == 2 * m + c && m < M) gemv_store(T[c][m], T[c ^ 1][m], m, ncol[c], N, bias, res, Y, ldy, ymap, epi);
+            for (int i = 0; i < 8; i++)
+                if (sb0 + i < nsb) S = fmaf(dv[i], xv[i], S);
+            T = T + S;
+        }
+        const float other = __shfl_xor(T, 1, WAVE);
+        if (m < M) gemv_store(T, other, m, column(c), N, bias, res, Y, ldy, ymap, epi);
+    }
 }
+
+// Launch of a matrix-vector call: two workgroups per CU, more where the outputs' x would not fit
+// 64 KB of LDS (so that two still share a CU); ONE where a workgroup's items fit one pass, with as
+// many threads as they take: activations straight from global memory then, beside the weights
+// (through LDS the 3584 x 3584 projection takes 5.7 us instead of 5.1).  grid = 0: one pair of
+// columns would not fit.
+struct gemv_shape {
+    int grid, threads;
+    size_t lds;
+    bool one;
+};
+static gemv_shape gemv_launch_shape(int wtype, int mr, int64_t N, int64_t K) {
+    const int64_t nsb = K / 256, pairs = N / 2, per_pair = mr * nsb * 8;
+    int64_t fixed = mr * (K + nsb * 36);
+    if (fixed + per_pair > 64 * 1024) return {0, 0, 0, false};
+    const int64_t room = (64 * 1024 - fixed) / per_pair;
+    const int64_t g = std::min(pairs, std::max<int64_t>(2 * device_cu_count(), (pairs + room - 1) / room));
+    const int64_t most = (pairs + g - 1) / g, lanes = 4 * most * nsb;
+    const int threads = gemv_threads(wtype, mr);
+    const bool one = lanes <= threads;
+    if (one) fixed = mr * nsb * 4;
+    return {(int)g, one ? (int)((lanes + 63) / 64 * 64) : threads, (size_t)(fixed + most * per_pair), one};
+}
+static int gemv_rows(int M) { return M <= 2 ? M : DFX_GEMV_M; }
 
 template <int WT>
 static int launch_gemv(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
-                       float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
-    // waves per pair: one per pass of 16 super-blocks, up to 16 (a workgroup per pair); one
-    // pass: four pairs per workgroup, one wave each
-    const int passes = (K / 256 + 15) / 16;
-    const bool split = passes > 1 && (K / 256 + 7) / 8 <= GEMV_MAX_CHUNKS;
-    const int ws = split ? std::min(passes, 16) : 1;
-    const dim3 grid((unsigned)(split ? N / 2 : (N / 2 + 3) / 4)), block((unsigned)(split ? 64 * ws : 256));
+                       float * y, int64_t ldy, const int32_t * ymap, const gemv_shape & s, hipStream_t st, dfx_epi epi) {
     const uint8_t * W = (const uint8_t *)w;
     const uint8_t * A = (const uint8_t *)act;
-#define GEMV_CASE(mr, sp) hipLaunchKernelGGL((k_gemv<WT, mr, sp>), grid, block, 0, st, W, N, K, A, M, bias, res, y, ldy, ymap, epi)
-#define GEMV_WS(mr) if (split) GEMV_CASE(mr, true); else GEMV_CASE(mr, false)
-    switch (M) {
-        case 1: GEMV_WS(1); break;
-        case 2: GEMV_WS(2); break;
-        default: GEMV_WS(4); break;
+#define GEMV_CASE(mr, one) hipLaunchKernelGGL((k_gemv<WT, mr, one>), dim3((unsigned)s.grid), dim3((unsigned)s.threads), \
+                                              s.lds, st, W, N, K, A, M, bias, res, y, ldy, ymap, epi)
+#define GEMV_ONE(mr) if (s.one) GEMV_CASE(mr, true); else GEMV_CASE(mr, false)
+    switch (gemv_rows(M)) {
+        case 1: GEMV_ONE(1); break;
+        case 2: GEMV_ONE(2); break;
+        default: GEMV_ONE(4); break;
     }
-#undef GEMV_WS
+#undef GEMV_ONE
 #undef GEMV_CASE
     DFX_CHECK_LAUNCH("dfx_gemm (matrix-vector)");
     return DFX_OK;
@@ -3052,16 +3064,15 @@ int dfx_gemm_ex(int wtype, const void * w, int64_t N, int64_t K, const void * ac
     if (M == 0) return DFX_OK;
     hipStream_t st = (hipStream_t)stream;
     const int n = (int)N, k = (int)K, m = (int)M;
-    // the matrix-vector kernels (unless a tile is forced) where they beat the matrix-core
-    // kernels: one row; two Q4_K rows; up to DFX_GEMV_M rows of a matrix of at most
-    // 4096 x 4096 (measured at the LLaDA-8B shapes: the integer dot products grow with the
-    // rows, the matrix-core kernels' time does not below 32 rows)
-    const bool gemv_rows = m == 1 || (m == 2 && wtype == DFX_TYPE_Q4_K) || (m <= DFX_GEMV_M && N * K <= 4096 * 4096);
-    if (gemv_rows && N % 32 == 0 && (wtype == DFX_TYPE_Q4_K || wtype == DFX_TYPE_Q6_K) &&
-        !forced_tile(wtype == DFX_TYPE_Q4_K ? 0 : 1).on) {
-        return wtype == DFX_TYPE_Q4_K ? launch_gemv<DFX_TYPE_Q4_K>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi)
-                                      : launch_gemv<DFX_TYPE_Q6_K>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
-    }
+    // the matrix-vector kernels (unless a tile is forced) up to DFX_GEMV_M rows: the same bits as
+    // the matrix-core kernels, whose time does not fall below 32 rows (at four rows, us, against
+    // them: LLaDA-8B gate|up 18 / 25, down 14 / 20, O 7.6 / 10.2, the Q6_K head 99 / 130)
+    const bool quads = (wtype == DFX_TYPE_Q4_K || wtype == DFX_TYPE_Q6_K) && m <= DFX_GEMV_M && N % 32 == 0 &&
+                       !forced_tile(wtype == DFX_TYPE_Q4_K ? 0 : 1).on;
+    if (const gemv_shape s = quads ? gemv_launch_shape(wtype, gemv_rows(m), N, K) : gemv_shape{}; s.grid)
+        return wtype == DFX_TYPE_Q4_K
+                   ? launch_gemv<DFX_TYPE_Q4_K>(w, n, k, act, m, bias, residual, y, ldy, ymap, s, st, epi)
+                   : launch_gemv<DFX_TYPE_Q6_K>(w, n, k, act, m, bias, residual, y, ldy, ymap, s, st, epi);
     switch (wtype) {
         case DFX_TYPE_Q4_K: return dispatch_q4k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
         case DFX_TYPE_Q6_K: return dispatch_q6k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
