@@ -5,8 +5,8 @@
 // Replaces ggml_mul_mat(W, X) of the reference graph (src/diffuse-graph.cpp:61-63,
 // 122, 136-140, 154 and the cached twins 451-453, 556, 570-574, 587).
 //
-// Quantised weights (Q4_K, Q6_K, Q8_0) run the "exact" kernel k_mmq, which
-// reproduces GGML's CPU dot products (ggml_vec_dot_q4_K_q8_K / q6_K_q8_K /
+// Quantised weights (Q4_K, Q6_K, Q8_0) run "exact" kernels (the first form is k_mmq), which
+// reproduce GGML's CPU dot products (ggml_vec_dot_q4_K_q8_K / q6_K_q8_K /
 // q8_0_q8_0): integer products summed exactly per block, then scaled and
 // accumulated in float in increasing K order, in the same order as the CPU
 // oracle:
@@ -1733,6 +1733,223 @@ k_q6k_w(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict
 }
 
 // ---------------------------------------------------------------------------
+// Q8_0 weights over more than a few rows
+// ---------------------------------------------------------------------------
+// Wave: 32 columns x TM row tiles of 32; workgroup: four waves side by side over 128 columns.  Sums
+// and their order: as k_mmq (isum of each 32-element block exact; x = d_w*isum; S = fma(d_a, x, S);
+// chunk sums T = T + S).
+//
+// What bounds it: the VALU, with two operations per output and block (16 each per lane and tile)
+// against 64 matrix-core cycles.  Everything else is kept off it and off the LDS that feeds it:
+// the activation scale of a row is read by the fma itself from the lane that holds it (DPP
+// row_newbcast: lane i of each 16 lanes loads the scale of the row that register i stands for,
+// four blocks in one 16-byte load), where k_mmq reads 16 scales a lane and block from LDS; the
+// activation tile goes global -> LDS by `buffer_load ... lds` one step of 128 ahead (rows of 128
+// bytes, chunk c of row r at slot c ^ (r & 7) ^ (r >> 3 & 3)), and so do the weights: loaded straight
+// into registers, 16 bytes of 32 columns at once, they kept the address path busy for longer than
+// all else takes (Q|K|V at 768 rows 238 us instead of 191 with 32-row tiles).  Integer sums do not depend on the
+// order, so both operands take elements 16 hl + 8 s .. + 7 of a block for MFMA s and lane half hl.
+// LLaDA-8B, us, before (k_mmq) -> after: Q|K|V 203 -> 147 at 768 rows, 79 -> 72 at 256, 47 -> 40 at 64;
+// gate|up 372 -> 282, 140 -> 121, 64 -> 50; down 221 -> 181, 127 -> 95, 128 -> 104; O 77 -> 65, 45 -> 34, 45 -> 35.
+template <int I>
+__device__ __forceinline__ void fmac_rows8(float16v & S, float da, const float (&x)[16]) {
+    // S[I + j] = fma(da of lane I + j of this lane's 16, x[I + j], S[I + j]); the wait states are for a da that
+    // a VALU instruction has just written
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %8, %9 row_newbcast:%c17 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %8, %10 row_newbcast:%c18 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %8, %11 row_newbcast:%c19 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %8, %12 row_newbcast:%c20 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %4, %8, %13 row_newbcast:%c21 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %5, %8, %14 row_newbcast:%c22 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %6, %8, %15 row_newbcast:%c23 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %7, %8, %16 row_newbcast:%c24 row_mask:0xf bank_mask:0xf"
+        : "+v"(S[I]), "+v"(S[I + 1]), "+v"(S[I + 2]), "+v"(S[I + 3]), "+v"(S[I + 4]), "+v"(S[I + 5]), "+v"(S[I + 6]),
+          "+v"(S[I + 7])
+        : "v"(da), "v"(x[I]), "v"(x[I + 1]), "v"(x[I + 2]), "v"(x[I + 3]), "v"(x[I + 4]), "v"(x[I + 5]), "v"(x[I + 6]),
+          "v"(x[I + 7]), "n"(I), "n"(I + 1), "n"(I + 2), "n"(I + 3), "n"(I + 4), "n"(I + 5), "n"(I + 6), "n"(I + 7));
+}
+
+template <int TM>
+__global__ void __launch_bounds__(256, 2)
+k_q8_w(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
+       const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
+       int n_tiles, int m_tiles, dfx_epi epi) {
+#pragma clang fp contract(off)
+    constexpr int BM = 32 * TM, NA = BM / 16;   // rows; 1 KB copies per wave and step (64 rows: 16 KB)
+    static_assert(TM >= 1 && TM <= 3, "row tiles");
+    __shared__ __attribute__((aligned(1024))) half_t As0[BM * 128], As1[BM * 128];   // [64 elements][row][64]
+    __shared__ __attribute__((aligned(1024))) uint8_t Ws0[128 * 128], Ws1[128 * 128];   // [column][128 quants]
+    auto aslot = [&](auto stage) __attribute__((always_inline)) -> half_t * {
+        if constexpr (decltype(stage)::value == 0) return As0;
+        else return As1;
+    };
+    auto wslot = [&](auto stage) __attribute__((always_inline)) -> uint8_t * {
+        if constexpr (decltype(stage)::value == 0) return Ws0;
+        else return Ws1;
+    };
+    const int L = blockIdx.x, xcd = L & 7, jj = L >> 3;
+    const int ty = jj % m_tiles, tx = 8 * (jj / m_tiles) + xcd;
+    if (tx >= n_tiles) return;
+    const int tid = threadIdx.x, lane = tid & 63, hl = lane >> 5, l32 = lane & 31;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = tx * 128, m0 = ty * BM;
+    const int n_kt = K >> 7;
+    const int64_t row_bytes = (int64_t)(K >> 8) * SB_Q8_0;
+    const act_layout Lay = act_layout_of(CONV_Q8_0, M, K);
+    // resources from the tile's first row: offsets inside its rows stay below 2^32
+    const __amdgpu_buffer_rsrc_t rW =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(W + n0 * row_bytes), 0, 0xFFFFFFFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(act + Lay.q + (int64_t)m0 * K * 2), 0, 0xFFFFFFFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rD = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(act + Lay.d + (int64_t)m0 * (K / 32) * 4), 0, 0xFFFFFFFF, 0x00020000);
+
+    uint32_t off_a[6], off_d[3], off_q[4];
+    const int r8 = lane >> 3;
+#pragma unroll
+    for (int j = 0; j < NA; j++) {   // copy c: rows 8 (c % (BM / 8)) .. + 7 of 64-element half c / (BM / 8)
+        const int c = NA * wv + j, sub = c / (BM / 8), rb = c % (BM / 8);
+        const int row = min(8 * rb + r8, M - 1 - m0);   // rows past the end repeat the last (not stored)
+        off_a[j] = (uint32_t)row * (uint32_t)(2 * K) + sub * 128 + (((lane & 7) ^ r8 ^ (rb & 3)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+        off_d[i] = (uint32_t)min(32 * i + tile_row(lane & 15, lane), M - 1 - m0) * (uint32_t)(K / 32 * 4);
+#pragma unroll
+    for (int j = 0; j < 4; j++)      // the wave's own columns, 8 per copy
+        off_q[j] = (uint32_t)min(32 * wv + 8 * j + r8, N - 1 - n0) * (uint32_t)row_bytes + 16 +
+                   (((lane & 7) ^ r8 ^ j) << 4);
+    const uint32_t off_w = (uint32_t)min(wv * 32 + l32, N - 1 - n0) * (uint32_t)row_bytes;
+
+    float4v da_st[2][3];
+    uint2 dw_st[2];
+    auto issue = [&](auto stage, int kt_req) __attribute__((always_inline)) {
+        constexpr int h = decltype(stage)::value;   // the step's parity: its half of the super-block
+        const int kt = min(kt_req, n_kt - 2 + h), sb = kt >> 1;
+#pragma unroll
+        for (int j = 0; j < NA; j++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, (lds_ptr)(aslot(stage) + (NA * wv + j) * 512), 16, off_a[j],
+                                                     kt * 256, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, (lds_ptr)(wslot(stage) + (4 * wv + j) * 1024), 16, off_q[j],
+                                                     sb * SB_Q8_0 + 128 * h, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        dw_st[h] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rW, off_w + 8 * h, sb * SB_Q8_0, 0));
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+            da_st[h][i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rD, off_d[i], kt * 16, 0));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int AFTER_A = 1 + TM;   // register loads of a step, issued after its copies
+
+    float16v S[TM], T[TM];
+    const float16v zero16 = {};
+#pragma unroll
+    for (int i = 0; i < TM; i++) { S[i] = zero16; T[i] = zero16; }
+    const int f = (l32 & 7) ^ (l32 >> 3);
+    const uint32_t C64 = opaque(0x64646464u);
+
+    auto step = [&](auto stage, int kt) __attribute__((always_inline)) {
+        constexpr int h = decltype(stage)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        // this step's copies done, and every LDS read of the previous step before the barrier
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm(AFTER_A, 0));
+        barrier_only();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(std::integral_constant<int, h ^ 1>{}, kt + 1);
+        const half_t * As = aslot(stage);
+        // tile-blocks in order (block b, row tile i): the MFMAs of one stand between the two halves of
+        // the flush of the same tile's block before, so that the matrix cores and the VALU work at
+        // the same time; operands are read one tile-block ahead, weights converted one block ahead
+        float16v P[2][TM];
+        half8 a[2][2], w[2][2];
+        u32x4 raw;
+        auto read = [&](int b, int i, half8 (&d)[2]) __attribute__((always_inline)) {
+            const half_t * p = As + (b >> 1) * (BM * 64) + (32 * i + l32) * 64;
+            const int c = 4 * (b & 1) + 2 * hl;
+            d[0] = *(const half8 *)(p + ((c ^ f) << 3));
+            d[1] = *(const half8 *)(p + (((c + 1) ^ f) << 3));
+        };
+        auto read_w = [&](int b) __attribute__((always_inline)) {
+            raw = *(const u32x4 *)(wslot(stage) + (32 * wv + l32) * 128 + (((2 * b + hl) ^ f) << 4));
+        };
+        auto convert = [&](half8 (&d)[2]) __attribute__((always_inline)) {
+            // q + 128 in the mantissa of 1024: 1024 + q + 128, less 1152
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                u32x4 pk;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const uint32_t v = raw[2 * s + e] ^ 0x80808080u;
+                    pk[2 * e] = __builtin_amdgcn_perm(C64, v, 0x04010400u);
+                    pk[2 * e + 1] = __builtin_amdgcn_perm(C64, v, 0x04030402u);
+                }
+                const half8 off = {(half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f,
+                                   (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f};
+                d[s] = __builtin_bit_cast(half8, pk) + off;
+            }
+        };
+        read_w(0);
+        read(0, 0, a[0]);
+        convert(w[0]);
+#pragma unroll
+        for (int b = 0; b <= 4; b++) {
+            const uint32_t dp = b - 1 < 2 ? dw_st[h].x : dw_st[h].y;
+            const float dw = h2f((uint16_t)(((b - 1) & 1) ? dp >> 16 : dp & 0xFFFFu));
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                const int u = (b * TM + i) & 1;
+                float x[16];
+                if (i == 0 && b < 3) read_w(b + 1);
+                if (b * TM + i + 1 < 4 * TM) read(i + 1 < TM ? b : b + 1, i + 1 < TM ? i + 1 : 0, a[u ^ 1]);
+                if (b < 4) {
+                    P[b & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u][0], w[b & 1][0], zero16, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (b > 0) {
+#pragma unroll
+                    for (int r = 0; r < 16; r++) x[r] = dw * P[(b - 1) & 1][i][r];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (b < 4) {
+                    P[b & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u][1], w[b & 1][1], P[b & 1][i], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (b > 0) {
+                    fmac_rows8<0>(S[i], da_st[h][i][b - 1], x);
+                    fmac_rows8<8>(S[i], da_st[h][i][b - 1], x);
+                }
+                if (i == TM - 1 && b < 3) convert(w[(b + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    issue(std::integral_constant<int, 0>{}, 0);
+    constexpr int CHUNK = DFX_DOT_CHUNK / 128;
+    for (int c0 = 0; c0 < n_kt; c0 += CHUNK) {
+        const int c1 = min(c0 + CHUNK, n_kt);
+        for (int kt = c0; kt < c1; kt += 2) {
+            step(std::integral_constant<int, 0>{}, kt);
+            step(std::integral_constant<int, 1>{}, kt + 1);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+            T[i] = T[i] + S[i];
+            S[i] = zero16;
+        }
+    }
+    // the copies issued past the last step still land in this workgroup's LDS
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm(0, 0));
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        __builtin_amdgcn_sched_barrier(0);
+        epilogue_tile(T[i], m0 + i * 32, n0 + wv * 32 + l32, M, N, bias, res, Y, ldy, ymap, nullptr, 0, lane, epi);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // F16 weights
 // ---------------------------------------------------------------------------
 template <int TM>
@@ -2332,6 +2549,16 @@ static int launch_mmq(const void * w, int N, int K, const void * act, int M, con
     return DFX_OK;
 }
 
+template <int TM>
+static int launch_q8_w(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
+                       float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
+    const int n_tiles = (N + 127) / 128, m_tiles = (M + 32 * TM - 1) / (32 * TM);
+    hipLaunchKernelGGL((k_q8_w<TM>), dim3((unsigned)(8 * ((n_tiles + 7) / 8) * m_tiles)), dim3(256), 0, st,
+                       (const uint8_t *)w, N, K, (const uint8_t *)act, M, bias, res, y, ldy, ymap, n_tiles, m_tiles, epi);
+    DFX_CHECK_LAUNCH("dfx_gemm q8_0");
+    return DFX_OK;
+}
+
 template <int TM, int TN, int D, int NWV = 4>
 static int launch_q4k(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
                       float * y, int64_t ldy, const int32_t * ymap, float * ws, hipStream_t st, int * defer,
@@ -2720,19 +2947,38 @@ static int pick_tm(int M, int max_tm) {
     return best;
 }
 
-// Q8_0: one 32-row tile per workgroup.  The per-32-element block flush keeps three
-// f32 totals per output in registers, and wider row tiles spill them (measured on
-// MI355X: 2-5x slower with 64 or 96 rows per workgroup at M = 96..768).
-template <int WT>
-static int dispatch_mmq(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
-                        float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
-    // 64-row tiles (each converted weight feeds two MFMAs) where their grid still gives every
-    // CU two workgroups; else 32-row tiles (same-box A/B over the LLaDA-8B projections: gate|up
-    // at 256 / 768 rows and Q|K|V at 768 rows 7-21 % faster with 64 rows, the narrower grids
-    // 0-35 % slower)
-    if ((int64_t)((N + 127) / 128) * ((M + 63) / 64) >= 2 * device_cu_count())
-        return launch_mmq<WT, 2>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
-    return launch_mmq<WT, 1>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+// Row tiles of a Q8_0 GEMM, by the time that each choice would take: full rounds of as many
+// workgroups as share the chip (three a CU of 32-row tiles, two of the larger ones) and a last one by
+// how many of them a CU carries; us per K step of 128, measured at N = 12288 and 4096.  Larger tiles
+// convert a weight for more rows and read it once for more MFMAs (1.0 / 0.69 / 0.61 in time per
+// row), smaller ones leave fewer CUs idle.  LLaDA-8B, 768 / 256 / 64 rows: Q|K|V 96 / 64 / 32-row
+// tiles, down 96 / 32 / 32, gate|up 96 / 64 / 64; the attention block at 768 rows 494 -> 427.
+// A single row tile of a matrix wide enough for more than one workgroup a CU stays with k_mmq, which has
+// no copies to wait for (Dream-7B gate|up at 32 rows 58 us against 63).
+static int dispatch_q8(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
+                       float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
+    static const struct { int per_cu; double us[3]; } form[] = {
+        {3, {1.04, 1.85, 2.35}}, {2, {1.37, 2.25, 0.0}}, {2, {1.97, 2.97, 0.0}}};
+    const int64_t n_tiles = (N + 127) / 128, cus = 256;
+    if (M <= 32 && n_tiles > cus)
+        return launch_mmq<DFX_TYPE_Q8_0, 1>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+    int best = 1;
+    double best_us = 1e30;
+    for (int tm = 1; tm <= 3; tm++) {
+        const auto & f = form[tm - 1];
+        const int64_t n = n_tiles * ((M + 32 * tm - 1) / (32 * tm)), slots = f.per_cu * cus;
+        const int64_t rest = n % slots;
+        const double us = (double)(n / slots) * f.us[f.per_cu - 1] + (rest ? f.us[(rest + cus - 1) / cus - 1] : 0.0);
+        if (us < best_us) {
+            best_us = us;
+            best = tm;
+        }
+    }
+    switch (best) {
+        case 1: return launch_q8_w<1>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+        case 2: return launch_q8_w<2>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+        default: return launch_q8_w<3>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -3076,7 +3322,7 @@ int dfx_gemm_ex(int wtype, const void * w, int64_t N, int64_t K, const void * ac
     switch (wtype) {
         case DFX_TYPE_Q4_K: return dispatch_q4k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
         case DFX_TYPE_Q6_K: return dispatch_q6k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
-        case DFX_TYPE_Q8_0: return dispatch_mmq<DFX_TYPE_Q8_0>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
+        case DFX_TYPE_Q8_0: return dispatch_q8(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
         case DFX_TYPE_F16:
             switch (f16_choice c = f16_choose(m, n, k, ws ? ws_bytes : 0); c.tiles) {
                 case F16_192x128: return launch_f16_w<2, 2, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);

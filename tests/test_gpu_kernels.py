@@ -216,6 +216,19 @@ def test_gemm_q6k_tiles_and_split_bit_exact(gpu, tile, N, K, M):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), rel_l2(got, ref)
 
 
+@pytest.mark.parametrize("N,K,M", [
+    (1, 256, 1), (100, 512, 33), (1000, 2304, 31),          # 32-row tiles; a chunk of one super-block
+    (4095, 4352, 129), (12281, 256, 250),                   # 64-row tiles: one and two a CU
+    (12281, 256, 380), (33000, 256, 20)])                   # 96-row tiles; one row tile of a wide matrix
+def test_gemm_q8_0_row_tiles_bit_exact(gpu, N, K, M):
+    """Q8_0 over every row tile of the dispatch, with ragged rows and columns: the oracle's bits."""
+    raw = quant(dfx.TYPE_Q8_0, N, K)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    got = gpu_gemm(dfx.TYPE_Q8_0, raw, N, K, X)
+    ref = O.mul_mat(dfx.TYPE_Q8_0, raw, N, K, X)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32)), rel_l2(got, ref)
+
+
 @pytest.mark.parametrize("N,K,M", [(1000, 4096, 33), (4096, 4096, 288), (4096, 12288, 64), (4096, 4096, 768)])
 def test_gemm_f16_matches_oracle(gpu, N, K, M):
     """F16: exact f16 products accumulated by MFMA in f32 (the oracle sums in f64)."""
