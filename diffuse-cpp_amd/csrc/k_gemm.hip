@@ -2494,12 +2494,21 @@ static int launch_f16_w(const void * w, int N, int K, const void * act, int M, c
     return DFX_OK;
 }
 
+// dfx_gemm_noalloc's split-K workspace: one round of 256 workgroups of 192 x 256 partial sums, the
+// largest split that the F16 rule below takes at up to 768 rows of the models' shapes.
+#define DFX_GEMM_SCRATCH_BYTES (48u << 20)
+
 // Tiles and K slices of an F16 GEMM over more than 256 rows, by the time that each choice would
 // take: rounds over the CUs (one workgroup each) x K steps of 32 x the tile's measured time a step
 // with cold weights, and for split K the slices' traffic at 4 TB/s and the reduction's launch.
 // k_gemm_f16's own tiles (128 x 128, two workgroups per CU) are among the choices: at 512 rows of
 // N = 12288 they take 82 us against 88 (192 x 256).  Up to 256 rows they are the better ones at
 // most shapes (N = 24576: 93 us against 109 at 256 rows, 67 against 76 at 128).
+//
+// The slices set the order of the f32 sums, so calls whose workspace holds DFX_GEMM_SCRATCH_BYTES
+// or dfx_gemm_ws_bytes must choose alike: no wide form takes partial sums beyond the former, and
+// f16_splits stays within it by itself (it doubles S below 256 workgroups of at most 128 x 128, so
+// it ends at 510 of them: 32 MiB).
 enum f16_tiles { F16_128x128, F16_192x128, F16_192x256, F16_256x256, F16_192x384 };
 struct f16_choice {
     f16_tiles tiles;
@@ -2516,8 +2525,9 @@ static f16_choice f16_choose(int64_t M, int64_t N, int64_t K, size_t ws_bytes) {
     f16_choice best{F16_128x128, s0};
     double best_us = steps / s0 * (n0 <= 256 ? 0.45 : n0 <= 512 ? 0.68 : 0.68 * 1.15 * n0 / 512) + slices_us(s0);
     if (M <= 256) return best;
+    const size_t room = std::min<size_t>(ws_bytes, DFX_GEMM_SCRATCH_BYTES);
     for (const auto & f : form)
-        for (int S = 1; S <= f.max_s && (S == 1 || (size_t)S * M * N * sizeof(float) <= ws_bytes); S *= 2) {
+        for (int S = 1; S <= f.max_s && (S == 1 || (size_t)S * M * N * sizeof(float) <= room); S *= 2) {
             const int64_t n = (N + f.bn - 1) / f.bn * ((M + f.bm - 1) / f.bm) * S;
             const double us = (double)((n + 255) / 256) * steps / S * f.us + slices_us(S);
             if (us < best_us) {
@@ -3403,7 +3413,6 @@ extern "C" int dfx_gemm_rope(int wtype, const void * w, int64_t N, int64_t K, co
 // code never passes the array's name to a kernel (in host code it is only a stand-in
 // symbol): the device address comes from hipGetSymbolAddress, looked up once per device on
 // that device's first call and kept in scratch_ptr[device].
-#define DFX_GEMM_SCRATCH_BYTES (32u << 20)
 static __device__ __align__(256) uint8_t scratch[DFX_GEMM_SCRATCH_BYTES];
 
 #define DFX_MAX_DEVICES 64
@@ -3437,19 +3446,9 @@ extern "C" int dfx_gemm_noalloc(int wtype, const void * w, int64_t N, int64_t K,
     // Quantised weights: the chunk sums are added in chunk order whether K is split or not,
     // so a workspace too small for the split dfx_gemm would choose only makes the dispatch
     // keep K whole, with the same bits.  F16: the slice count decides the f32 summation
-    // order, so the split dfx_gemm would choose must fit the array.  F32 and Q8_0 use no
+    // order; f16_choose takes no split that the array does not hold.  F32 and Q8_0 use no
     // workspace.
     const size_t full = M > 0 && N > 0 && K > 0 ? dfx_gemm_ws_bytes(M, N, K) : 0;
-    if (wtype == DFX_TYPE_F16 && M > 0 && N > 0 && K > 0 && K % 256 == 0) {
-        const int S = f16_splits(pick_tm((int)std::min<int64_t>(M, INT32_MAX), 4), M, N, K, full);
-        const size_t need = S > 1 ? (size_t)S * M * N * sizeof(float) : 0;
-        if (need > DFX_GEMM_SCRATCH_BYTES) {
-            dfx_set_error("dfx_gemm_noalloc: the F16 split's partial sums (%d slices, %zu bytes) exceed the %u-byte "
-                          "scratch (M=%lld N=%lld K=%lld)", S, need, DFX_GEMM_SCRATCH_BYTES, (long long)M,
-                          (long long)N, (long long)K);
-            return DFX_ERR_ARG;
-        }
-    }
     const size_t ws_bytes = std::min<size_t>(full, DFX_GEMM_SCRATCH_BYTES);
     return dfx_gemm_ex(wtype, w, N, K, act, M, bias, residual, y, N, nullptr, scratch_ptr[dev], ws_bytes, stream,
                        nullptr, nullptr);

@@ -180,11 +180,10 @@ int dfx_gemm_rope(int wtype, const void * w, int64_t N, int64_t K, const void * 
 int dfx_gemm_force_tile(int wtype, const char * spec);
 
 /* dfx_gemm without a workspace argument and without any allocation: the split-K partial
- * sums go to a library-held device array of 32 MiB per GPU (held from the library's load to
+ * sums go to a library-held device array of 48 MiB per GPU (held from the library's load to
  * process end).  Quantised weights whose split would need more (M * N * ceil(K / 2048) * 4
- * bytes) keep K whole, which gives the same bits; an F16 split that would not fit is refused
- * with DFX_ERR_ARG (the split rule needs at most 16 MiB).  Same kernels and the same bits as
- * dfx_gemm with a workspace.  The first call on a device may be made under stream capture
+ * bytes) keep K whole, which gives the same bits; the F16 split rule takes no more than the
+ * array holds, with any workspace.  The same bits as dfx_gemm with a workspace.  The first call on a device may be made under stream capture
  * (it looks the array's address up with the thread's capture mode relaxed).  Calls on one GPU
  * share that array: calls that overlap in time on one GPU (several streams or host threads)
  * race; serialise them.  No counterpart in the reference: for callers that cannot allocate

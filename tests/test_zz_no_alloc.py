@@ -41,6 +41,11 @@ def _run(typ, w, ab, N, K, M, res, noalloc):
     [(dfx.TYPE_Q4_K, 4096, 12288, 64, True), (dfx.TYPE_Q4_K, 1024, 4096, 20, False)],
     [(dfx.TYPE_Q6_K, 2048, 12288, 100, False), (dfx.TYPE_Q6_K, 640, 4096, 33, True)],
     [(dfx.TYPE_F16, 4096, 12288, 64, False), (dfx.TYPE_F16, 1000, 4096, 33, False)],
+    # F16 over more than 256 rows: the tile choice sets the slices, hence the order of the f32 sums
+    # (48 MiB of partial sums at 768 rows; at 1100 rows the array's size bounds the choice)
+    [(dfx.TYPE_F16, 4096, 12288, 768, True), (dfx.TYPE_F16, 4096, 12288, 600, False)],
+    [(dfx.TYPE_F16, 4096, 4096, 768, False), (dfx.TYPE_F16, 3584, 18944, 650, False)],
+    [(dfx.TYPE_F16, 4096, 12288, 1100, False)],
 ])
 def test_noalloc_gemm_matches_dfx_gemm(gpu, calls):
     for typ, N, K, M, residual in calls:
