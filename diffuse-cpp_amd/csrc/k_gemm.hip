@@ -2476,15 +2476,16 @@ static int launch_f16(const void * w, int N, int K, const void * act, int M, con
     return DFX_OK;
 }
 
+// K steps of 32 in each of S slices of a wide form: a multiple of 8 (K is one of 256 elements)
+static int64_t f16_w_steps(int64_t n_kt, int64_t S) { return (n_kt + 8 * S - 1) / (8 * S) * 8; }
+
 template <int WM, int WN, int TM, int TN>
 static int launch_f16_w(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
                         float * y, int64_t ldy, const int32_t * ymap, void * ws, int S, hipStream_t st, int * defer,
                         dfx_epi epi) {
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
     const int n_tiles = (N + BN - 1) / BN, m_tiles = (M + BM - 1) / BM;
-    // K steps per slice: a multiple of 8 (K is one of 256 elements)
-    const int n_kt = K / 32, per = (n_kt + 8 * S - 1) / (8 * S) * 8;
-    S = (n_kt + per - 1) / per;
+    const int per = (int)f16_w_steps(K / 32, S);
     const int per_pass = 8 * ((n_tiles + 7) / 8) * m_tiles;
     hipLaunchKernelGGL((k_gemm_f16_w<WM, WN, TM, TN>), dim3((unsigned)(per_pass * S)), dim3(64 * WM * WN), 0, st,
                        (const uint8_t *)w, N, K, (const uint8_t *)act, M, bias, res, y, ldy, ymap, n_tiles, m_tiles,
@@ -2494,42 +2495,80 @@ static int launch_f16_w(const void * w, int N, int K, const void * act, int M, c
     return DFX_OK;
 }
 
+// M tile (32 * TM rows) with the least row padding, larger tiles on ties.
+static int pick_tm(int M, int max_tm) {
+    int best = 1, best_pad = 1 << 30;
+    for (int t = 1; t <= max_tm; t++) {
+        const int pad = ((M + 32 * t - 1) / (32 * t)) * 32 * t;
+        if (pad <= best_pad) { best = t; best_pad = pad; }
+    }
+    return best;
+}
+
 // dfx_gemm_noalloc's split-K workspace: one round of 256 workgroups of 192 x 256 partial sums, the
 // largest split that the F16 rule below takes at up to 768 rows of the models' shapes.
 #define DFX_GEMM_SCRATCH_BYTES (48u << 20)
 
-// Tiles and K slices of an F16 GEMM over more than 256 rows, by the time that each choice would
-// take: rounds over the CUs (one workgroup each) x K steps of 32 x the tile's measured time a step
-// with cold weights, and for split K the slices' traffic at 4 TB/s and the reduction's launch.
-// k_gemm_f16's own tiles (128 x 128, two workgroups per CU) are among the choices: at 512 rows of
-// N = 12288 they take 82 us against 88 (192 x 256).  Up to 256 rows they are the better ones at
-// most shapes (N = 24576: 93 us against 109 at 256 rows, 67 against 76 at 128).
+// Compute units of the current device (cached per device).
+static int device_cu_count() {
+    static std::atomic<int> cached[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int v = cached[dev].load(std::memory_order_relaxed);
+    if (!v) {
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
+        cached[dev].store(v, std::memory_order_relaxed);
+    }
+    return v;
+}
+
+// Tiles and K slices of an F16 GEMM.  Up to 256 rows k_gemm_f16 with the row tile of least padding
+// is the better one at most shapes (N = 24576: 93 us against 109 at 256 rows, 67 against 76 at 128).
+// Above, by the time that each choice would take: K steps of 32 times the tile's measured time a
+// step (medians over 13 shapes, cold weights) with up to one workgroup per CU, up to two, and for
+// every CU-count of workgroups beyond; for split K the slices' traffic at 4 TB/s and the reduction's
+// launch; and 3 us more for a wide tile, whose ring fills before the first product.  Workgroups are
+// counted as launched: a wide form's column tiles go round the eight XCDs, so where their number is
+// no multiple of eight the XCDs that have one more fill first (N = 4608 at 1200 rows: 252 tiles of
+// 192 x 128, but 35 on some XCDs' 32 CUs: 86 us; priced so, 192 x 256 tiles take 76).  Over
+// 22 row counts x 13 shapes the choice takes 0.3 % longer than the fastest form on average; k_gemm_f16's
+// row tile is priced as it is launched (at 385 rows of N = 3584, K = 18944 its 32-row tiles take
+// 166 us, 192 x 256 in four slices 103).
 //
 // The slices set the order of the f32 sums, so calls whose workspace holds DFX_GEMM_SCRATCH_BYTES
 // or dfx_gemm_ws_bytes must choose alike: no wide form takes partial sums beyond the former, and
 // f16_splits stays within it by itself (it doubles S below 256 workgroups of at most 128 x 128, so
 // it ends at 510 of them: 32 MiB).
-enum f16_tiles { F16_128x128, F16_192x128, F16_192x256, F16_256x256, F16_192x384 };
+enum f16_tiles { F16_ROWS, F16_192x128, F16_192x256, F16_256x256, F16_192x384 };
 struct f16_choice {
     f16_tiles tiles;
-    int S;
+    int n;           // F16_ROWS: row tiles of 32 per workgroup; else K slices
 };
+struct f16_step { double one, two, more; };   // us
 static f16_choice f16_choose(int64_t M, int64_t N, int64_t K, size_t ws_bytes) {
-    static const struct { f16_tiles tiles; int bm, bn, max_s; double us; } form[] = {
-        {F16_192x128, 192, 128, 4, 0.47}, {F16_192x256, 192, 256, 4, 0.72},
-        {F16_256x256, 256, 256, 1, 0.85}, {F16_192x384, 192, 384, 1, 1.05}};
-    const double steps = (double)K / 32;
-    auto slices_us = [&](int S) { return S > 1 ? S * 8e-6 * (double)M * (double)N / 4.0 + 3.0 : 0.0; };
-    const int s0 = f16_splits(4, M, N, K, ws_bytes);
-    const double n0 = (double)((N + 127) / 128 * ((M + 127) / 128) * s0);
-    f16_choice best{F16_128x128, s0};
-    double best_us = steps / s0 * (n0 <= 256 ? 0.45 : n0 <= 512 ? 0.68 : 0.68 * 1.15 * n0 / 512) + slices_us(s0);
-    if (M <= 256) return best;
+    static const f16_step row_us[4] = {{0.265, 0.285, 0.147}, {0.315, 0.38, 0.218}, {0.39, 0.50, 0.31}, {0.48, 0.61, 0.38}};
+    static const struct { f16_tiles tiles; int bm, bn, max_s; f16_step us; } wide[] = {
+        {F16_192x128, 192, 128, 4, {0.43, 0.81, 0.40}}, {F16_192x256, 192, 256, 4, {0.64, 1.40, 0.67}},
+        {F16_256x256, 256, 256, 1, {0.72, 1.60, 0.80}}, {F16_192x384, 192, 384, 1, {0.87, 1.93, 0.93}}};
+    const int tm = pick_tm((int)std::min<int64_t>(M, INT32_MAX), 4);
+    f16_choice best{F16_ROWS, tm};
+    // a wide form's copies take 32-bit offsets inside a tile's rows
+    if (M <= 256 || K > (1 << 22)) return best;
+    const int64_t cus = device_cu_count(), n_kt = K / 32;
+    auto step_us = [&](const f16_step & u, int64_t wgs) {
+        return wgs <= cus ? u.one : wgs <= 2 * cus ? u.two : u.more * (double)((wgs + cus - 1) / cus);
+    };
+    auto slices_us = [&](int S) { return S > 1 ? S * 8e-6 * (double)M * (double)N / 4.0 + 5.0 : 0.0; };
+    const int s0 = f16_splits(tm, M, N, K, ws_bytes);
+    double best_us = (double)n_kt / s0 * step_us(row_us[tm - 1], (N + 127) / 128 * ((M + 32 * tm - 1) / (32 * tm)) * s0) +
+                     slices_us(s0);
     const size_t room = std::min<size_t>(ws_bytes, DFX_GEMM_SCRATCH_BYTES);
-    for (const auto & f : form)
+    for (const auto & f : wide)
         for (int S = 1; S <= f.max_s && (S == 1 || (size_t)S * M * N * sizeof(float) <= room); S *= 2) {
-            const int64_t n = (N + f.bn - 1) / f.bn * ((M + f.bm - 1) / f.bm) * S;
-            const double us = (double)((n + 255) / 256) * steps / S * f.us + slices_us(S);
+            const int64_t per = f16_w_steps(n_kt, S);
+            if ((n_kt + per - 1) / per != S) continue;
+            const int64_t wgs = 8 * (((N + f.bn - 1) / f.bn + 7) / 8) * ((M + f.bm - 1) / f.bm) * S;
+            const double us = 3.0 + (double)per * step_us(f.us, wgs) + slices_us(S);
             if (us < best_us) {
                 best_us = us;
                 best = {f.tiles, S};
@@ -2646,19 +2685,6 @@ static int launch_q4k_w(const void * w, int N, int K, const void * act, int M, c
     DFX_CHECK_LAUNCH("dfx_gemm q4_k");
     if (ws && !halves) return reduce_or_defer(ws, chunks, M, N, bias, res, y, ldy, ymap, st, defer, epi);
     return DFX_OK;
-}
-
-// Compute units of the current device (cached per device).
-static int device_cu_count() {
-    static std::atomic<int> cached[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    int v = cached[dev].load(std::memory_order_relaxed);
-    if (!v) {
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-        cached[dev].store(v, std::memory_order_relaxed);
-    }
-    return v;
 }
 
 // Whole tiles for the first n_full workgroups, half tiles after them.  Taken where a grid of
@@ -2945,16 +2971,6 @@ static int dispatch_q4k(const void * w, int N, int K, const void * act, int M, c
         default: return launch_q4k<1, 1, 2>(w, N, K, act, M, bias, res, y, ldy, ymap, wsf, st, defer, epi);
     }
 #undef Q4K_CASE
-}
-
-// M tile (32 * TM rows) with the least row padding, larger tiles on ties.
-static int pick_tm(int M, int max_tm) {
-    int best = 1, best_pad = 1 << 30;
-    for (int t = 1; t <= max_tm; t++) {
-        const int pad = ((M + 32 * t - 1) / (32 * t)) * 32 * t;
-        if (pad <= best_pad) { best = t; best_pad = pad; }
-    }
-    return best;
 }
 
 // Row tiles of a Q8_0 GEMM, by the time that each choice would take: full rounds of as many
@@ -3333,20 +3349,22 @@ int dfx_gemm_ex(int wtype, const void * w, int64_t N, int64_t K, const void * ac
         case DFX_TYPE_Q4_K: return dispatch_q4k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
         case DFX_TYPE_Q6_K: return dispatch_q6k(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
         case DFX_TYPE_Q8_0: return dispatch_q8(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
-        case DFX_TYPE_F16:
-            switch (f16_choice c = f16_choose(m, n, k, ws ? ws_bytes : 0); c.tiles) {
-                case F16_192x128: return launch_f16_w<2, 2, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
-                case F16_192x256: return launch_f16_w<2, 4, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
-                case F16_256x256: return launch_f16_w<2, 4, 4, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
-                case F16_192x384: return launch_f16_w<2, 4, 3, 3>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.S, st, defer, epi);
-                case F16_128x128: break;
+        case DFX_TYPE_F16: {
+            const f16_choice c = f16_choose(m, n, k, ws ? ws_bytes : 0);
+            switch (c.tiles) {
+                case F16_192x128: return launch_f16_w<2, 2, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.n, st, defer, epi);
+                case F16_192x256: return launch_f16_w<2, 4, 3, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.n, st, defer, epi);
+                case F16_256x256: return launch_f16_w<2, 4, 4, 2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.n, st, defer, epi);
+                case F16_192x384: return launch_f16_w<2, 4, 3, 3>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, c.n, st, defer, epi);
+                case F16_ROWS: break;
             }
-            switch (pick_tm(m, 4)) {
+            switch (c.n) {
                 case 1: return launch_f16<1>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
                 case 2: return launch_f16<2>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
                 case 3: return launch_f16<3>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
                 default: return launch_f16<4>(w, n, k, act, m, bias, residual, y, ldy, ymap, ws, ws_bytes, st, defer, epi);
             }
+        }
         case DFX_TYPE_F32:
             if (m <= 32) return launch_f32<1>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);
             return launch_f32<2>(w, n, k, act, m, bias, residual, y, ldy, ymap, st, epi);

@@ -242,9 +242,10 @@ def test_gemm_f16_matches_oracle(gpu, N, K, M):
 
 @pytest.mark.parametrize("N,K,M", [
     (12281, 768, 384),                       # 192 x 128 tiles
-    (4096, 4096, 768), (24571, 256, 300),    # the same with split K; 192 x 256
-    (4090, 8192, 600),                       # 192 x 256 with split K
-    (24570, 512, 500), (24576, 256, 700)])   # 256 x 256; 192 x 384
+    (4096, 4096, 768), (3001, 4096, 322),    # the same in two and four K slices
+    (8191, 256, 769), (4090, 8192, 600),     # 192 x 256, and in four K slices
+    (24570, 512, 500), (24576, 256, 700),    # 256 x 256; 192 x 384
+    (24571, 256, 300), (3584, 512, 385)])    # few K steps: the 64- and 32-row tiles of the smaller form
 def test_gemm_f16_wide_tiles(gpu, N, K, M):
     """F16 over more than 256 rows: the wide tiles, with ragged rows and columns and with split K,
     against f64 sums of the same f16 values.  A sum of K exact products in f32 is off by at most
@@ -354,7 +355,8 @@ def oracle_swiglu(g, u):
     (dfx.TYPE_Q4_K, 2688, 3584, 24, None),   # wide, few rows: two-wave tiles, split K, SwiGLU in the reduction
     (dfx.TYPE_Q6_K, 512, 12288, 40, "2x1s"), (dfx.TYPE_Q4_K, 512, 12288, 40, "ks"), (dfx.TYPE_Q4_K, 512, 3584, 70, "k"), (dfx.TYPE_Q4_K, 768, 4096, 50, "k4"),
     (dfx.TYPE_Q6_K, 512, 4096, 66, "2x1n"), (dfx.TYPE_Q8_0, 512, 4096, 33, None),
-    (dfx.TYPE_F16, 512, 4096, 33, None), (dfx.TYPE_F16, 5600, 256, 257, None),   # the second: wide tiles
+    (dfx.TYPE_F16, 512, 4096, 33, None), (dfx.TYPE_F16, 5600, 256, 257, None),
+    (dfx.TYPE_F16, 2816, 1024, 353, None), (dfx.TYPE_F16, 2816, 2304, 353, None),   # wide tiles; with split K
     (dfx.TYPE_F32, 256, 512, 20, None)])
 def test_gemm_swiglu_epilogue_bit_exact(gpu, typ, F, K, M, tile):
     """dfx_gemm_swiglu on an interleaved gate|up matrix: the same bits as the plain GEMM's
@@ -415,7 +417,8 @@ def rope_row_order(H, Hkv, hd):
     (dfx.TYPE_Q4_K, 4, 2, 128, 3584, 50, "ks", True), (dfx.TYPE_Q4_K, 6, 2, 64, 4096, 40, "k", True), (dfx.TYPE_Q4_K, 4, 2, 128, 4096, 74, "k2s", True),
     (dfx.TYPE_Q6_K, 4, 2, 128, 4096, 66, "2x1s", True), (dfx.TYPE_Q6_K, 4, 4, 64, 2048, 100, "2x1n", False),
     (dfx.TYPE_Q8_0, 4, 2, 128, 2048, 33, None, True), (dfx.TYPE_F16, 4, 1, 128, 2048, 45, None, True),
-    (dfx.TYPE_F16, 32, 32, 128, 256, 300, None, True),   # wide tiles
+    (dfx.TYPE_F16, 32, 32, 128, 256, 300, None, True),
+    (dfx.TYPE_F16, 32, 32, 128, 768, 384, None, True),   # wide tiles
     (dfx.TYPE_F32, 2, 1, 64, 512, 20, None, False)])
 def test_gemm_rope_epilogue_bit_exact(gpu, typ, H, Hkv, hd, K, M, tile, bias):
     """dfx_gemm_rope on the row-permuted Q|K|V matrix stores the same q, K-cache and
