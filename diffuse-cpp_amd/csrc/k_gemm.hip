@@ -2975,24 +2975,30 @@ static int dispatch_q4k(const void * w, int N, int K, const void * act, int M, c
 
 // Row tiles of a Q8_0 GEMM, by the time that each choice would take: full rounds of as many
 // workgroups as share the chip (three a CU of 32-row tiles, two of the larger ones) and a last one by
-// how many of them a CU carries; us per K step of 128, measured at N = 12288 and 4096.  Larger tiles
-// convert a weight for more rows and read it once for more MFMAs (1.0 / 0.69 / 0.61 in time per
-// row), smaller ones leave fewer CUs idle.  LLaDA-8B, 768 / 256 / 64 rows: Q|K|V 96 / 64 / 32-row
+// how many of them a CU carries; us per K step of 128, fitted to 13 shapes x 25 row counts.  Larger tiles
+// convert a weight for more rows and read it once for more MFMAs, smaller ones leave fewer CUs idle.
+// The larger tiles' workgroups are counted as launched, column tiles padded to a multiple of eight:
+// their number going round the XCDs, the XCDs that have one more column run out of CUs first (N = 4608
+// at 640 rows: 252 tiles of 96 rows are 35 on four XCDs' 32 CUs, 81 us; 64-row tiles 62).  Three
+// 32-row tiles on a CU even that out, so those are counted as they are (N = 3584, K = 18944 at 288
+// rows 176 us, 64-row tiles 186).  LLaDA-8B, 768 / 256 / 64 rows: Q|K|V 96 / 64 / 32-row
 // tiles, down 96 / 32 / 32, gate|up 96 / 64 / 64; the attention block at 768 rows 494 -> 427.
 // A single row tile of a matrix wide enough for more than one workgroup a CU stays with k_mmq, which has
-// no copies to wait for (Dream-7B gate|up at 32 rows 58 us against 63).
+// no copies to wait for (Dream-7B gate|up at 32 rows 58 us against 62, at 16 rows 55 / 58, at one 57 / 52).
 static int dispatch_q8(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
                        float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
     static const struct { int per_cu; double us[3]; } form[] = {
-        {3, {1.04, 1.85, 2.35}}, {2, {1.37, 2.25, 0.0}}, {2, {1.97, 2.97, 0.0}}};
-    const int64_t n_tiles = (N + 127) / 128, cus = 256;
-    if (M <= 32 && n_tiles > cus)
+        {3, {1.0, 1.4, 2.2}}, {2, {1.3, 2.15, 0.0}}, {2, {1.9, 2.95, 0.0}}};
+    const int64_t n_tiles = (N + 127) / 128, cus = device_cu_count();
+    // a wide tile's copies take 32-bit offsets inside its rows
+    if ((M <= 32 && n_tiles > cus) || K > (1 << 24))
         return launch_mmq<DFX_TYPE_Q8_0, 1>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
     int best = 1;
     double best_us = 1e30;
     for (int tm = 1; tm <= 3; tm++) {
         const auto & f = form[tm - 1];
-        const int64_t n = n_tiles * ((M + 32 * tm - 1) / (32 * tm)), slots = f.per_cu * cus;
+        const int64_t cols = tm == 1 ? n_tiles : 8 * ((n_tiles + 7) / 8);
+        const int64_t n = cols * ((M + 32 * tm - 1) / (32 * tm)), slots = f.per_cu * cus;
         const int64_t rest = n % slots;
         const double us = (double)(n / slots) * f.us[f.per_cu - 1] + (rest ? f.us[(rest + cus - 1) / cus - 1] : 0.0);
         if (us < best_us) {

@@ -217,9 +217,11 @@ def test_gemm_q6k_tiles_and_split_bit_exact(gpu, tile, N, K, M):
 
 
 @pytest.mark.parametrize("N,K,M", [
-    (1, 256, 1), (100, 512, 33), (1000, 2304, 31),          # 32-row tiles; a chunk of one super-block
-    (4095, 4352, 129), (12281, 256, 250),                   # 64-row tiles: one and two a CU
-    (12281, 256, 380), (33000, 256, 20)])                   # 96-row tiles; one row tile of a wide matrix
+    (1, 256, 1), (100, 512, 33), (1000, 2304, 31), (4095, 4352, 129),   # 32-row tiles; a chunk of one super-block
+    (4095, 4352, 300), (12281, 256, 250), (12281, 4352, 250),           # 64-row tiles: one and two a CU
+    (12281, 256, 380), (12281, 2304, 380),                              # 96-row tiles
+    (4608, 2304, 640),           # 64-row tiles where 96-row ones would need a second workgroup on some CUs
+    (33000, 256, 20), (33000, 4352, 20), (33000, 2304, 32)])            # one row tile of a wide matrix
 def test_gemm_q8_0_row_tiles_bit_exact(gpu, N, K, M):
     """Q8_0 over every row tile of the dispatch, with ragged rows and columns: the oracle's bits."""
     raw = quant(dfx.TYPE_Q8_0, N, K)
