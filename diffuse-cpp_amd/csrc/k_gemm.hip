@@ -5,8 +5,7 @@
 // Replaces ggml_mul_mat(W, X) of the reference graph (src/diffuse-graph.cpp:61-63,
 // 122, 136-140, 154 and the cached twins 451-453, 556, 570-574, 587).
 //
-// Quantised weights (Q4_K, Q6_K, Q8_0) run "exact" kernels (the first form is k_mmq), which
-// reproduce GGML's CPU dot products (ggml_vec_dot_q4_K_q8_K / q6_K_q8_K /
+// Quantised weights (Q4_K, Q6_K, Q8_0) run "exact" kernels, which reproduce GGML's CPU dot products (ggml_vec_dot_q4_K_q8_K / q6_K_q8_K /
 // q8_0_q8_0): integer products summed exactly per block, then scaled and
 // accumulated in float in increasing K order, in the same order as the CPU
 // oracle:
@@ -21,14 +20,11 @@
 // rounding difference into whole quantisation steps that grow over the layers;
 // exactness here is what keeps the logits on the CPU path's trajectory.
 //
-// F16 weights run k_gemm_f16, and k_gemm_f16_w where more rows fill its wider tiles: f16 x f16 products (exact) accumulated by MFMA in
-// f32 (GGML accumulates them in f32/f64 SIMD lanes in its own order).
+// F16 weights run k_gemm_f16, and k_gemm_f16_w where more rows fill its wider tiles: f16 x f16
+// products (exact) accumulated by MFMA in f32 (GGML accumulates them in f32/f64 SIMD lanes in its
+// own order).
 //
-// Tiling: workgroup = 4 waves splitting 128 weight rows (32 each); TM tiles of
-// 32 activation rows per wave.  K step = 128 (half a super-block).  Raw weight
-// bytes and the f16 activation tile are staged in LDS; every wave converts its
-// own 32 weight rows into B fragments in registers; the next step's global loads
-// are issued before the current step's MFMAs.
+// Tiling: each kernel says its own.  A K step is 128 (half a super-block) unless it says otherwise.
 #include "dfx_device.h"
 
 #include <algorithm>
@@ -43,21 +39,11 @@
 
 // Raw bytes per weight row per K step (half super-block), as 16-byte chunks.
 template <int WT> struct WT_;
-template <> struct WT_<DFX_TYPE_Q4_K> { static constexpr int CH = 5,  SB = SB_Q4_K; };
-template <> struct WT_<DFX_TYPE_Q6_K> { static constexpr int CH = 8,  SB = SB_Q6_K; };
 template <> struct WT_<DFX_TYPE_Q8_0> { static constexpr int CH = 9,  SB = SB_Q8_0; };
 template <> struct WT_<DFX_TYPE_F16>  { static constexpr int CH = 16, SB = SB_F16; };
 
 // Byte offset inside a super-block of chunk c of half h.
 template <int WT> __device__ __forceinline__ int chunk_off(int c, int h);
-template <> __device__ __forceinline__ int chunk_off<DFX_TYPE_Q4_K>(int c, int h) {
-    return c == 0 ? 0 : 16 + 64 * h + 16 * (c - 1);                // header | qs half
-}
-template <> __device__ __forceinline__ int chunk_off<DFX_TYPE_Q6_K>(int c, int h) {
-    return c < 4 ? 64 * h + 16 * c                                  // ql half
-         : c < 6 ? 128 + 32 * h + 16 * (c - 4)                      // qh half
-         : c == 6 ? 192 : 208;                                      // scales | d
-}
 template <> __device__ __forceinline__ int chunk_off<DFX_TYPE_Q8_0>(int c, int h) {
     return c == 0 ? 0 : 16 + 128 * h + 16 * (c - 1);               // d[8] | qs half
 }
@@ -125,13 +111,6 @@ struct stage {
         }
     }
 };
-
-__device__ __forceinline__ half8 to_half8(const int v[8]) {
-    half8 r;
-#pragma unroll
-    for (int j = 0; j < 8; j++) r[j] = (half_t)v[j];   // |v| <= 2048, or a power-of-two multiple: exact
-    return r;
-}
 
 // Row of register r of a 32x32 MFMA tile held by `lane` (its column is lane % 32).
 __device__ __forceinline__ int tile_row(int r, int lane) { return 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3); }
@@ -286,223 +265,96 @@ __device__ __forceinline__ void epilogue_tile(const V16 & acc, int m0, int n, in
 }
 
 // ---------------------------------------------------------------------------
-// Exact kernel for quantised weights
+// Q8_0 weights, one row tile of the widest matrices
 // ---------------------------------------------------------------------------
-template <int WT, int TM>
+// 32 rows x 128 columns per workgroup, four waves side by side; weights and activations go through
+// registers to LDS between two barriers a K step.  k_q8_w is faster wherever more rows or fewer
+// columns come with it; over up to 32 rows of more columns than a workgroup a CU takes, several of
+// these workgroups share a CU and cover each other's barriers.
 __global__ void __launch_bounds__(256, 2)
-k_mmq(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
-      const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
-      dfx_epi epi) {
+k_mmq_q8(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
+         const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
+         dfx_epi epi) {
 #pragma clang fp contract(off)
-    constexpr int BM = TM * 32, BN = 128, WSTR = wstride<WT>();
-    constexpr bool KQ = WT != DFX_TYPE_Q8_0;     // Q8_K activations: d per 256, bsums per 16
-    constexpr int BSTR = 24;                     // LDS halves per row of 16 block sums
+    constexpr int BM = 32, BN = 128, WSTR = wstride<DFX_TYPE_Q8_0>();
     __shared__ __attribute__((aligned(16))) uint8_t Ws[BN * WSTR];
     __shared__ __attribute__((aligned(16))) half_t As[BM * ASTR];
-    __shared__ __attribute__((aligned(16))) float Ad[BM * 4];          // KQ: [BM]; Q8_0: [4][BM]
-    __shared__ __attribute__((aligned(16))) half_t Abs[KQ ? BM * BSTR : 8];
+    __shared__ __attribute__((aligned(16))) float Ad[4 * BM];          // [block of the K step][row]
 
     const int tid = threadIdx.x, lane = tid & 63, wn = tid >> 6;
     const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
     const int n_kt = K / BK;
-    const int64_t row_bytes = (int64_t)(K >> 8) * WT_<WT>::SB;
-    const act_layout Lay = act_layout_of(KQ ? CONV_Q8_K : CONV_Q8_0, M, K);
+    const int64_t row_bytes = (int64_t)(K >> 8) * SB_Q8_0;
+    const act_layout Lay = act_layout_of(CONV_Q8_0, M, K);
     const half_t * Aq = (const half_t *)(act + Lay.q);
     const float * Adg = (const float *)(act + Lay.d);
-    const half_t * Absg = (const half_t *)(act + Lay.bs);
 
-    stage<WT, BM, BN> st;
-    float dreg = 0.0f;                                  // KQ: d_a of row tid (tid < BM)
-    float4 dreg4 = make_float4(0, 0, 0, 0);             // Q8_0: d_a of the 4 blocks of the K step
-    uint4 bsreg = make_uint4(0, 0, 0, 0);               // KQ: 8 of the 16 block sums of row tid/2
-
-    auto load_meta = [&](int kt) {
-        const int sb = kt >> 1;
-        if (KQ) {
-            if ((kt & 1) == 0) {
-                if (tid < BM) dreg = (m0 + tid < M) ? Adg[(int64_t)(m0 + tid) * (K / 256) + sb] : 0.0f;
-                if (tid < 2 * BM) {
-                    const int r = tid >> 1, c = tid & 1;
-                    bsreg = (m0 + r < M) ? *(const uint4 *)(Absg + (int64_t)(m0 + r) * (K / 16) + sb * 16 + c * 8)
-                                         : make_uint4(0, 0, 0, 0);
-                }
-            }
-        } else if (tid < BM) {
+    stage<DFX_TYPE_Q8_0, BM, BN> st;
+    float4 dreg4 = make_float4(0, 0, 0, 0);                            // d_a of the 4 blocks of the K step
+    auto load_d = [&](int kt) {
+        if (tid < BM)
             dreg4 = (m0 + tid < M) ? *(const float4 *)(Adg + (int64_t)(m0 + tid) * (K / 32) + kt * 4)
                                    : make_float4(0, 0, 0, 0);
-        }
     };
-    auto store_meta = [&](int kt) {
-        if (KQ) {
-            if ((kt & 1) == 0) {
-                if (tid < BM) Ad[tid] = dreg;
-                if (tid < 2 * BM) *(uint4 *)(Abs + (tid >> 1) * BSTR + (tid & 1) * 8) = bsreg;
-            }
-        } else if (tid < BM) {
-            // [block][row]: a lane's four consecutive tile rows of one block are one 16-byte read
+
+    float16v P = {}, S = {}, T = {};
+    const uint8_t * wp = Ws + (wn * 32 + (lane & 31)) * WSTR;          // this lane's weight row
+    const int hl = lane >> 5;
+
+    st.load(W, N, row_bytes, Aq, M, K, n0, m0, 0, tid);
+    load_d(0);
+    for (int kt = 0; kt < n_kt; kt++) {
+        __syncthreads();
+        st.store(Ws, As, tid);
+        if (tid < BM) {
             Ad[tid] = dreg4.x;
             Ad[BM + tid] = dreg4.y;
             Ad[2 * BM + tid] = dreg4.z;
             Ad[3 * BM + tid] = dreg4.w;
         }
-    };
-
-    float16v P[TM], S1[TM], T1[TM];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) P[i][r] = S1[i][r] = T1[i][r] = 0.0f;
-
-    const uint8_t * wp = Ws + (wn * 32 + (lane & 31)) * WSTR;   // this lane's weight row
-    const int hl = lane >> 5;
-
-    st.load(W, N, row_bytes, Aq, M, K, n0, m0, 0, tid);
-    load_meta(0);
-    for (int kt = 0; kt < n_kt; kt++) {
-        __syncthreads();
-        st.store(Ws, As, tid);
-        store_meta(kt);
         __syncthreads();
         if (kt + 1 < n_kt) {
             st.load(W, N, row_bytes, Aq, M, K, n0, m0, kt + 1, tid);
-            load_meta(kt + 1);
+            load_d(kt + 1);
         }
         const int h = kt & 1;
 #pragma unroll
         for (int kk = 0; kk < BK / 16; kk++) {
             const int e = kk * 16 + 8 * hl;      // first of this lane's 8 K elements in the step
-            int u[8], u2[8];
-            if (WT == DFX_TYPE_Q4_K) {
-                int sc, mn;
-                q4k_scale_min(4 * h + (e >> 5), wp + 4, sc, mn);
-                const uint2 q = *(const uint2 *)(wp + 16 + 32 * (e >> 6) + (e & 31));
-                const int sh = 4 * ((e >> 5) & 1);
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    u[j] = sc * (int)((q.x >> (8 * j + sh)) & 15);
-                    u[4 + j] = sc * (int)((q.y >> (8 * j + sh)) & 15);
-                }
-            } else if (WT == DFX_TYPE_Q6_K) {
-                const int quarter = e >> 5, l = e & 31;
-                const uint2 lo = *(const uint2 *)(wp + l + 32 * (quarter & 1));
-                const uint2 hb = *(const uint2 *)(wp + 64 + l);
-                const int sc = (int8_t)wp[96 + 8 * h + 2 * quarter + (l >> 4)];
-                const int sl = 4 * (quarter >> 1), sh = 2 * quarter;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const uint32_t lw = j < 4 ? lo.x : lo.y, hw = j < 4 ? hb.x : hb.y;
-                    const int jj = j & 3;
-                    const int q6 = (int)(((lw >> (8 * jj + sl)) & 15) | (((hw >> (8 * jj + sh)) & 3) << 4));
-                    // q6 - 32 = 8*c + e with c in [-4, 3], e in [0, 7]
-                    u[j] = 8 * (sc * ((q6 >> 3) - 4));
-                    u2[j] = sc * (q6 & 7);
-                }
-            }
-            half8 b;
-            if (WT == DFX_TYPE_Q8_0) {
-                // int8 q as an exact f16 integer without conversions: q + 128 (the byte with its
-                // top bit flipped) becomes the mantissa of 0x6400 = 1024.0 (v_perm places two bytes
-                // beside 0x64 bytes), and one packed f16 add of -1152 leaves q
-                const uint2 qw = *(const uint2 *)(wp + 16 + e);
-                const uint32_t x0 = qw.x ^ 0x80808080u, x1 = qw.y ^ 0x80808080u;
-                const u32x4 pk = {__builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u),
-                                  __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u),
-                                  __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u),
-                                  __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u)};
-                const half8 off = {(half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f,
-                                   (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f};
-                b = __builtin_bit_cast(half8, pk) + off;
-            } else {
-                b = to_half8(u);
-            }
-            half8 b2;
-            if (WT == DFX_TYPE_Q6_K) b2 = to_half8(u2);
-#pragma unroll
-            for (int i = 0; i < TM; i++) {
-                const half8 a = *(const half8 *)(As + (i * 32 + (lane & 31)) * ASTR + e);
-                P[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, P[i], 0, 0, 0);
-                if (WT == DFX_TYPE_Q6_K) P[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b2, P[i], 0, 0, 0);
-            }
-            if (WT == DFX_TYPE_Q8_0 && (kk & 1)) {
-                // a 32-element block is complete: sum += isum * (d_w * d_a)
+            // int8 q as an exact f16 integer without conversions: q + 128 (the byte with its
+            // top bit flipped) becomes the mantissa of 0x6400 = 1024.0 (v_perm places two bytes
+            // beside 0x64 bytes), and one packed f16 add of -1152 leaves q
+            const uint2 qw = *(const uint2 *)(wp + 16 + e);
+            const uint32_t x0 = qw.x ^ 0x80808080u, x1 = qw.y ^ 0x80808080u;
+            const u32x4 pk = {__builtin_amdgcn_perm(x0, 0x64646464u, 0x00050004u),
+                              __builtin_amdgcn_perm(x0, 0x64646464u, 0x00070006u),
+                              __builtin_amdgcn_perm(x1, 0x64646464u, 0x00050004u),
+                              __builtin_amdgcn_perm(x1, 0x64646464u, 0x00070006u)};
+            const half8 off = {(half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f,
+                               (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f, (half_t)-1152.0f};
+            const half8 a = *(const half8 *)(As + (lane & 31) * ASTR + e);
+            P = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, __builtin_bit_cast(half8, pk) + off, P, 0, 0, 0);
+            if (kk & 1) {
+                // a 32-element block is complete: S = fma(d_a, d_w*isum, S)
                 const int bl = kk >> 1;
                 const float dw = h2f(*(const uint16_t *)(wp + 2 * (4 * h + bl)));
+                // registers 4g..4g+3 hold rows 8g + 4(lane/32) + 0..3: one 16-byte read each
+                float dav[16];
 #pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    // registers 4g..4g+3 hold rows 8g + 4(lane/32) + 0..3: one 16-byte read each
-                    // from the [block][row] layout of Ad
-                    float dav[16];
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const float4 d4 = *(const float4 *)(Ad + bl * BM + i * 32 + 8 * g + 4 * hl);
-                        dav[4 * g] = d4.x; dav[4 * g + 1] = d4.y; dav[4 * g + 2] = d4.z; dav[4 * g + 3] = d4.w;
-                    }
-                    flush_d(S1[i], P[i], dw, dav);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) P[i][r] = 0.0f;
+                for (int g = 0; g < 4; g++) {
+                    const float4 d4 = *(const float4 *)(Ad + bl * BM + 8 * g + 4 * hl);
+                    dav[4 * g] = d4.x; dav[4 * g + 1] = d4.y; dav[4 * g + 2] = d4.z; dav[4 * g + 3] = d4.w;
                 }
+                flush_d(S, P, dw, dav);
+                P = float16v{};
             }
         }
-        if (!KQ && ((kt + 1) % (DFX_DOT_CHUNK / BK) == 0 || kt + 1 == n_kt)) {
-            // chunk complete: T = T + S
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) { T1[i][r] = T1[i][r] + S1[i][r]; S1[i][r] = 0.0f; }
-        }
-        if (KQ && h == 1) {
-            // super-block complete
-            if (WT == DFX_TYPE_Q4_K) {
-                // msum = sum_j m_j * (bsum_{2j} + bsum_{2j+1}) as a 16-deep product:
-                // B[k][n] = m_{k/2}, k = 8*(lane/32) + t
-                int mv[8];
-#pragma unroll
-                for (int t = 0; t < 8; t += 2) {
-                    int sc, mn;
-                    q4k_scale_min(4 * hl + t / 2, wp + 4, sc, mn);
-                    mv[t] = mv[t + 1] = mn;
-                }
-                const half8 bm = to_half8(mv);
-                const float dw = h2f(*(const uint16_t *)(wp + 0)), dmw = h2f(*(const uint16_t *)(wp + 2));
-#pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    const half8 a = *(const half8 *)(Abs + (i * 32 + (lane & 31)) * BSTR + 8 * hl);
-                    float16v Q;
-#pragma unroll
-                    for (int r = 0; r < 16; r++) Q[r] = 0.0f;
-                    Q = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bm, Q, 0, 0, 0);
-                    float dav[16];
-#pragma unroll
-                    for (int r = 0; r < 16; r++) dav[r] = Ad[i * 32 + tile_row(r, lane)];
-                    flush_dmin(S1[i], P[i], Q, dw, dmw, dav);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) P[i][r] = 0.0f;
-                }
-            } else {
-                const float dw = h2f(*(const uint16_t *)(wp + 112));
-#pragma unroll
-                for (int i = 0; i < TM; i++) {
-                    float dav[16];
-#pragma unroll
-                    for (int r = 0; r < 16; r++) dav[r] = Ad[i * 32 + tile_row(r, lane)];
-                    flush_d(S1[i], P[i], dw, dav);
-#pragma unroll
-                    for (int r = 0; r < 16; r++) P[i][r] = 0.0f;
-                }
-            }
-            if (((kt >> 1) + 1) % (DFX_DOT_CHUNK / 256) == 0 || kt + 1 == n_kt) {
-                // chunk complete: T = T + S
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) { T1[i][r] = T1[i][r] + S1[i][r]; S1[i][r] = 0.0f; }
-            }
+        if ((kt + 1) % (DFX_DOT_CHUNK / BK) == 0 || kt + 1 == n_kt) {   // chunk complete
+            T = T + S;
+            S = float16v{};
         }
     }
-
-    const int n = n0 + wn * 32 + (lane & 31);
-#pragma unroll
-    for (int i = 0; i < TM; i++) epilogue_tile(T1[i], m0 + i * 32, n, M, N, bias, res, Y, ldy, ymap, nullptr, 0, lane, epi);
+    epilogue_tile(T, m0, n0 + wn * 32 + (lane & 31), M, N, bias, res, Y, ldy, ymap, nullptr, 0, lane, epi);
 }
 
 // ---------------------------------------------------------------------------
@@ -1736,20 +1588,20 @@ k_q6k_w(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict
 // Q8_0 weights over more than a few rows
 // ---------------------------------------------------------------------------
 // Wave: 32 columns x TM row tiles of 32; workgroup: four waves side by side over 128 columns.  Sums
-// and their order: as k_mmq (isum of each 32-element block exact; x = d_w*isum; S = fma(d_a, x, S);
+// and their order: as k_mmq_q8 (isum of each 32-element block exact; x = d_w*isum; S = fma(d_a, x, S);
 // chunk sums T = T + S).
 //
 // What bounds it: the VALU, with two operations per output and block (16 each per lane and tile)
 // against 64 matrix-core cycles.  Everything else is kept off it and off the LDS that feeds it:
 // the activation scale of a row is read by the fma itself from the lane that holds it (DPP
 // row_newbcast: lane i of each 16 lanes loads the scale of the row that register i stands for,
-// four blocks in one 16-byte load), where k_mmq reads 16 scales a lane and block from LDS; the
+// four blocks in one 16-byte load), where k_mmq_q8 reads 16 scales a lane and block from LDS; the
 // activation tile goes global -> LDS by `buffer_load ... lds` one step of 128 ahead (rows of 128
 // bytes, chunk c of row r at slot c ^ (r & 7) ^ (r >> 3 & 3)), and so do the weights: loaded straight
 // into registers, 16 bytes of 32 columns at once, they kept the address path busy for longer than
 // all else takes (Q|K|V at 768 rows 238 us instead of 191 with 32-row tiles).  Integer sums do not depend on the
 // order, so both operands take elements 16 hl + 8 s .. + 7 of a block for MFMA s and lane half hl.
-// LLaDA-8B, us, before (k_mmq) -> after: Q|K|V 203 -> 147 at 768 rows, 79 -> 72 at 256, 47 -> 40 at 64;
+// LLaDA-8B, us, before (a 32- or 64-row form of k_mmq_q8) -> after: Q|K|V 203 -> 147 at 768 rows, 79 -> 72 at 256, 47 -> 40 at 64;
 // gate|up 372 -> 282, 140 -> 121, 64 -> 50; down 221 -> 181, 127 -> 95, 128 -> 104; O 77 -> 65, 45 -> 34, 45 -> 35.
 template <int I>
 __device__ __forceinline__ void fmac_rows8(float16v & S, float da, const float (&x)[16]) {
@@ -2587,14 +2439,12 @@ static int launch_f32(const void * w, int N, int K, const void * act, int M, con
     return DFX_OK;
 }
 
-template <int WT, int TM>
-static int launch_mmq(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
-                      float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
-    constexpr int BM = TM * 32, BN = 128;
-    const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM);
-    hipLaunchKernelGGL((k_mmq<WT, TM>), grid, dim3(256), 0, st, (const uint8_t *)w, N, K, (const uint8_t *)act, M,
-                       bias, res, y, ldy, ymap, epi);
-    DFX_CHECK_LAUNCH("dfx_gemm");
+static int launch_mmq_q8(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
+                         float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
+    const dim3 grid((N + 127) / 128, (M + 31) / 32);
+    hipLaunchKernelGGL(k_mmq_q8, grid, dim3(256), 0, st, (const uint8_t *)w, N, K, (const uint8_t *)act, M, bias, res, y,
+                       ldy, ymap, epi);
+    DFX_CHECK_LAUNCH("dfx_gemm q8_0");
     return DFX_OK;
 }
 
@@ -2983,7 +2833,7 @@ static int dispatch_q4k(const void * w, int N, int K, const void * act, int M, c
 // 32-row tiles on a CU even that out, so those are counted as they are (N = 3584, K = 18944 at 288
 // rows 176 us, 64-row tiles 186).  LLaDA-8B, 768 / 256 / 64 rows: Q|K|V 96 / 64 / 32-row
 // tiles, down 96 / 32 / 32, gate|up 96 / 64 / 64; the attention block at 768 rows 494 -> 427.
-// A single row tile of a matrix wide enough for more than one workgroup a CU stays with k_mmq, which has
+// A single row tile of a matrix wide enough for more than one workgroup a CU stays with k_mmq_q8, which has
 // no copies to wait for (Dream-7B gate|up at 32 rows 58 us against 62, at 16 rows 55 / 58, at one 57 / 52).
 static int dispatch_q8(const void * w, int N, int K, const void * act, int M, const float * bias, const float * res,
                        float * y, int64_t ldy, const int32_t * ymap, hipStream_t st, dfx_epi epi) {
@@ -2992,7 +2842,7 @@ static int dispatch_q8(const void * w, int N, int K, const void * act, int M, co
     const int64_t n_tiles = (N + 127) / 128, cus = device_cu_count();
     // a wide tile's copies take 32-bit offsets inside its rows
     if ((M <= 32 && n_tiles > cus) || K > (1 << 24))
-        return launch_mmq<DFX_TYPE_Q8_0, 1>(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
+        return launch_mmq_q8(w, N, K, act, M, bias, res, y, ldy, ymap, st, epi);
     int best = 1;
     double best_us = 1e30;
     for (int tm = 1; tm <= 3; tm++) {
