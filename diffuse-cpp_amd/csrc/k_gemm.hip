@@ -2875,13 +2875,17 @@ static int dispatch_q8(const void * w, int N, int K, const void * act, int M, co
 // exactly, in int32; the four lanes of a super-block add them (DPP quad permutes) and
 // x = d_w*isum (Q4_K: x = fma(-dmin_w, msum, x)) goes to LDS.  After one barrier a lane per
 // output runs the exact float order over all super-blocks: S = fma(d_a, x, S) in each chunk of 8,
-// T = T + S.
+// T = T + S; over more than two chunks a lane per output and chunk makes S first.
 //
 // What bounds it: HBM at the widest (5.5 TB/s over the vocab heads), below that the latency of the
-// first loads.  A wave per pair of columns, which this replaces, ran the chains wave-wide from
-// v_readlane and loaded and converted the activations for every pair.  One row, us, before -> after:
-// Dream-7B gate|up 21.0 -> 16.8, down 16.3 -> 13.2, Q4_K head 66.8 -> 55.7, Q6_K head 111 -> 84;
-// LLaDA-8B gate|up 16.0 -> 14.0, down 11.5 -> 10.3.
+// first loads and of what follows the last.  So a lane's first weights, activations and scales are
+// requested together, and no index is divided: the partition comes from the host, and t / nsb is a
+// multiplication (64-bit divisions for the partition alone cost 0.4-0.5 us of every call).
+// Against a wave per pair of columns, whose chains ran wave-wide from v_readlane and which loaded
+// and converted the activations for every pair, us: one row, Dream-7B gate|up 21.4 -> 16.8, down
+// 16.5 -> 11.8, Q4_K head 67 -> 54, Q6_K head 111 -> 85, LLaDA-8B gate|up 16.8 -> 14.0, down
+// 12.0 -> 9.7, 1536 x 512 3.2 -> 3.1; four rows, against the 32-row matrix-core tiles, LLaDA-8B
+// gate|up 25.7 -> 17.7, down 20.5 -> 13.6, O 10.3 -> 6.9, Dream-7B's Q6_K head 131 -> 117.
 __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }
@@ -2932,8 +2936,16 @@ __device__ __forceinline__ void gemv_store(float v, float w, int m, int n, int N
 }
 
 // Threads of a workgroup, two of which share a CU: 8 waves each leave 128 registers a lane, which
-// Q6_K over several rows overflows (the head at four rows 140 us with the spills, 118 with 6 waves).
+// Q6_K over several rows overflows (Dream-7B's head at four rows 140 us with the spills, 117 with 6 waves).
 constexpr int gemv_threads(int wt, int rows) { return wt == DFX_TYPE_Q6_K && rows > 1 ? 384 : 512; }
+
+// Partition of the column pairs: workgroup w takes pairs + (w < extra) of them; inv_nsb =
+// ceil(2^31 / nsb) divides t by the super-blocks of a row as the high word of (2 t + 1) * inv_nsb,
+// exactly while (2 t + 1) * 2 nsb < 2^32 (t is below 10240: an item's x alone takes 8 bytes of LDS).
+struct gemv_part {
+    int pairs, extra;
+    uint32_t inv_nsb;
+};
 
 // Raw weights of one item: a lane's share of a super-block of two columns.
 template <int WT> struct gemv_raw;
@@ -2944,16 +2956,20 @@ template <int WT, int MR, bool ONE>
 __global__ void __launch_bounds__(gemv_threads(WT, MR)) __attribute__((amdgpu_waves_per_eu(gemv_threads(WT, MR) / 128)))
 k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
        const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
-       dfx_epi epi) {
+       gemv_part part, dfx_epi epi) {
 #pragma clang fp contract(off)
     constexpr bool Q4 = WT == DFX_TYPE_Q4_K;
     constexpr int SB = Q4 ? SB_Q4_K : SB_Q6_K;
     extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
     const int tid = threadIdx.x, g = tid & 3;
     const int nsb = K >> 8, T4 = (int)blockDim.x >> 2;   // items per pass
-    const int p0 = (int)((int64_t)blockIdx.x * (N / 2) / gridDim.x);
-    const int ncol = 2 * ((int)((int64_t)(blockIdx.x + 1) * (N / 2) / gridDim.x) - p0);
+    const int wg = blockIdx.x, p0 = wg * part.pairs + min(wg, part.extra);
+    const int ncol = 2 * (part.pairs + (wg < part.extra ? 1 : 0));
     const int items = nsb * (ncol / 2);
+    // t / nsb
+    auto pair_of = [&](int t) __attribute__((always_inline)) -> int {
+        return (int)__umulhi(2 * (uint32_t)t + 1, part.inv_nsb);
+    };
     const int a_bytes = ONE ? 0 : MR * K, b_bytes = ONE ? 0 : MR * nsb * 32;
     u32x4 * as = (u32x4 *)gemv_lds;                           // [MR][4][nsb * 4]: piece i of group g
     uint2 * bs = (uint2 *)(gemv_lds + a_bytes);               // [MR][nsb * 4]: the group's sums
@@ -2984,7 +3000,7 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
     };
     // item t: pair t / nsb of the workgroup, super-block t % nsb (past the end: the last again)
     auto load = [&](int t_req, gemv_raw<WT> & r) __attribute__((always_inline)) {
-        const int t = min(t_req, items - 1), pl = t / nsb, sb = t - pl * nsb;
+        const int t = min(t_req, items - 1), pl = pair_of(t), sb = t - pl * nsb;
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const uint8_t * blk = W + (int64_t)column(2 * pl + c) * rb + (int64_t)sb * SB;
@@ -3005,15 +3021,24 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
             }
         }
     };
+    // ONE: the lane's activations and sums, requested with its weights
+    u32x4 a1[ONE ? MR : 1][4];
+    uint2 b1[ONE ? MR : 1];
     auto compute = [&](int t, const gemv_raw<WT> & r) __attribute__((always_inline)) {
-        const int pl = t / nsb, sb = t - pl * nsb;
+        const int pl = pair_of(t), sb = t - pl * nsb;
 #pragma unroll
         for (int m = 0; m < MR; m++) {
             u32x4 a[4];
+            uint2 b;
+            if constexpr (ONE) {
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-                a[i] = ONE ? piece(m, sb, g, i) : as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + g];
-            const uint2 b = ONE ? sums(m, sb, g) : bs[m * nsb * 4 + 4 * sb + g];
+                for (int i = 0; i < 4; i++) a[i] = a1[m][i];
+                b = b1[m];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; i++) a[i] = as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + g];
+                b = bs[m * nsb * 4 + 4 * sb + g];
+            }
             float x[2];
 #pragma unroll
             for (int c = 0; c < 2; c++) {
@@ -3060,23 +3085,43 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
     gemv_raw<WT> r0, r1;
     int t = tid >> 2;
     load(t, r0);
-    if constexpr (!ONE) {
-        for (int u = tid; u < MR * nsb * 16; u += (int)blockDim.x) {
-            const int m = u / (nsb * 16), v = u - m * nsb * 16, sb = v >> 4, gg = (v >> 2) & 3, i = v & 3;
-            as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + gg] = piece(m, sb, gg, i);
+    float d1[MR];
+    if constexpr (ONE) {
+        const int tc = min(t, items - 1), sb = tc - pair_of(tc) * nsb;
+#pragma unroll
+        for (int m = 0; m < MR; m++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) a1[m][i] = piece(m, sb, g, i);
+            b1[m] = sums(m, sb, g);
         }
-        for (int u = tid; u < MR * nsb * 4; u += (int)blockDim.x) {
-            const int m = u / (nsb * 4), v = u - m * nsb * 4;
-            bs[u] = sums(m, v >> 2, v & 3);
+#pragma unroll
+        for (int m = 0; m < MR; m++) d1[m] = ad[(int64_t)min(tid, nsb - 1) * Lay.mq + min(m, M - 1)];
+    } else {
+        for (int v = tid; v < nsb * 16; v += (int)blockDim.x) {
+            const int sb = v >> 4, gg = (v >> 2) & 3, i = v & 3;
+            u32x4 x[MR];
+#pragma unroll
+            for (int m = 0; m < MR; m++) x[m] = piece(m, sb, gg, i);
+#pragma unroll
+            for (int m = 0; m < MR; m++) as[(size_t)m * (K / 16) + i * (4 * nsb) + 4 * sb + gg] = x[m];
         }
-    }
-    for (int u = tid; u < MR * nsb; u += (int)blockDim.x) {
-        const int m = u / nsb, sb = u - m * nsb;
-        ds[u] = ad[(int64_t)sb * Lay.mq + min(m, M - 1)];
+        for (int v = tid; v < nsb * 4; v += (int)blockDim.x) {
+            uint2 x[MR];
+#pragma unroll
+            for (int m = 0; m < MR; m++) x[m] = sums(m, v >> 2, v & 3);
+#pragma unroll
+            for (int m = 0; m < MR; m++) bs[m * nsb * 4 + v] = x[m];
+        }
+        for (int sb = tid; sb < nsb; sb += (int)blockDim.x)
+#pragma unroll
+            for (int m = 0; m < MR; m++) ds[m * nsb + sb] = ad[(int64_t)sb * Lay.mq + min(m, M - 1)];
     }
     // (a quad's four lanes share its items, so quad_sum sees all of them or none)
     if constexpr (ONE) {
         if (t < items) compute(t, r0);
+        if (tid < nsb)
+#pragma unroll
+            for (int m = 0; m < MR; m++) ds[m * nsb + tid] = d1[m];
     } else {
         __syncthreads();
         for (; t < items; t += 2 * T4) {
@@ -3087,49 +3132,65 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
         }
     }
     __syncthreads();
-    for (int o = tid; o < MR * ncol; o += (int)blockDim.x) {   // ncol is even: o ^ 1 is the paired column of the same row
-        const int m = o / ncol, c = o - m * ncol;
-        const float * xr = xs + (size_t)m * nsb * ncol + c, * dr = ds + m * nsb;
-        float T = 0.0f;
-        for (int sb0 = 0; sb0 < nsb; sb0 += 8) {
-            float xv[8], dv[8], S = 0.0f;
+    // S of a chunk: lane (row m, column c) from super-block sb0
+    auto chunk = [&](const float * xr, const float * dr, int left) __attribute__((always_inline)) -> float {
+        float xv[8], dv[8], S = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int sb = min(sb0 + i, nsb - 1);
-                xv[i] = xr[sb * ncol];
-                dv[i] = dr[sb];
-            }
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (sb0 + i < nsb) S = fmaf(dv[i], xv[i], S);
-            T = T + S;
+        for (int i = 0; i < 8; i++) {
+            const int k = min(i, left - 1);
+            xv[i] = xr[k * ncol];
+            dv[i] = dr[k];
         }
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (i < left) S = fmaf(dv[i], xv[i], S);
+        return S;
+    };
+    const int nch = (nsb + 7) >> 3;
+    if (nch > 2) {   // a lane per output and chunk; S takes the place of the chunk's first x
+        for (int o = tid; o < MR * nch * ncol; o += (int)blockDim.x) {
+            const int q = o / ncol, c = o - q * ncol, m = MR == 1 ? 0 : q / nch, sb0 = 8 * (q - m * nch);
+            float * xr = xs + (size_t)(m * nsb + sb0) * ncol + c;
+            *xr = chunk(xr, ds + m * nsb + sb0, nsb - sb0);
+        }
+        __syncthreads();
+    }
+    for (int o = tid; o < MR * ncol; o += (int)blockDim.x) {   // ncol is even: o ^ 1 is the paired column of the same row
+        const int m = MR == 1 ? 0 : o / ncol, c = o - m * ncol;
+        const float * xr = xs + (size_t)m * nsb * ncol + c;
+        float T = 0.0f;
+        for (int sb0 = 0; sb0 < nsb; sb0 += 8)
+            T = T + (nch > 2 ? xr[sb0 * ncol] : chunk(xr + sb0 * ncol, ds + m * nsb + sb0, nsb - sb0));
         const float other = __shfl_xor(T, 1, WAVE);
         if (m < M) gemv_store(T, other, m, column(c), N, bias, res, Y, ldy, ymap, epi);
     }
 }
 
-// Launch of a matrix-vector call: two workgroups per CU, more where the outputs' x would not fit
-// 64 KB of LDS (so that two still share a CU); ONE where a workgroup's items fit one pass, with as
-// many threads as they take: activations straight from global memory then, beside the weights
-// (through LDS the 3584 x 3584 projection takes 5.7 us instead of 5.1).  grid = 0: one pair of
-// columns would not fit.
+// Launch of a matrix-vector call.  ONE where a workgroup's items fit one pass over two workgroups
+// per CU, each of them filling a wave (16 / nsb pairs) if there are so few (1536 x 512: 96 workgroups
+// 3.1 us, 512 of a quarter of a wave 3.6), with as many threads as the items take: activations
+// straight from global memory then, beside the weights.  Else the activations are staged, in up to
+// half of a CU's 160 KB; where the outputs' x needs more workgroups than two per CU, whole rounds of
+// them (N = 28672, K = 8192 at four rows: 1024 instead of 531, 33 us instead of 44).  grid = 0: one pair of
+// columns would not fit (K beyond 17 k at three or four rows, 34 k at two, 69 k at one).
+constexpr int64_t GEMV_LDS = 80 * 1024;
 struct gemv_shape {
     int grid, threads;
     size_t lds;
     bool one;
 };
 static gemv_shape gemv_launch_shape(int wtype, int mr, int64_t N, int64_t K) {
-    const int64_t nsb = K / 256, pairs = N / 2, per_pair = mr * nsb * 8;
-    int64_t fixed = mr * (K + nsb * 36);
-    if (fixed + per_pair > 64 * 1024) return {0, 0, 0, false};
-    const int64_t room = (64 * 1024 - fixed) / per_pair;
-    const int64_t g = std::min(pairs, std::max<int64_t>(2 * device_cu_count(), (pairs + room - 1) / room));
-    const int64_t most = (pairs + g - 1) / g, lanes = 4 * most * nsb;
+    const int64_t nsb = K / 256, pairs = N / 2, per_pair = mr * nsb * 8, slots = 2 * device_cu_count();
     const int threads = gemv_threads(wtype, mr);
-    const bool one = lanes <= threads;
-    if (one) fixed = mr * nsb * 4;
-    return {(int)g, one ? (int)((lanes + 63) / 64 * 64) : threads, (size_t)(fixed + most * per_pair), one};
+    if (4 * ((pairs + slots - 1) / slots) * nsb <= threads) {
+        const int64_t fill = std::max<int64_t>(1, 16 / nsb), g = std::min((pairs + fill - 1) / fill, slots);
+        const int64_t most = (pairs + g - 1) / g;
+        return {(int)g, (int)((4 * most * nsb + 63) / 64 * 64), (size_t)(mr * nsb * 4 + most * per_pair), true};
+    }
+    const int64_t fixed = mr * (K + nsb * 36), room = (GEMV_LDS - fixed) / per_pair;
+    if (GEMV_LDS < fixed + per_pair) return {0, 0, 0, false};
+    const int64_t g = std::min(pairs, (pairs + room * slots - 1) / (room * slots) * slots);
+    return {(int)g, threads, (size_t)(fixed + (pairs + g - 1) / g * per_pair), false};
 }
 static int gemv_rows(int M) { return M <= 2 ? M : DFX_GEMV_M; }
 
@@ -3138,8 +3199,10 @@ static int launch_gemv(const void * w, int N, int K, const void * act, int M, co
                        float * y, int64_t ldy, const int32_t * ymap, const gemv_shape & s, hipStream_t st, dfx_epi epi) {
     const uint8_t * W = (const uint8_t *)w;
     const uint8_t * A = (const uint8_t *)act;
+    const uint32_t nsb = (uint32_t)(K / 256);
+    const gemv_part part = {N / 2 / s.grid, N / 2 % s.grid, (0x80000000u + nsb - 1) / nsb};
 #define GEMV_CASE(mr, one) hipLaunchKernelGGL((k_gemv<WT, mr, one>), dim3((unsigned)s.grid), dim3((unsigned)s.threads), \
-                                              s.lds, st, W, N, K, A, M, bias, res, y, ldy, ymap, epi)
+                                              s.lds, st, W, N, K, A, M, bias, res, y, ldy, ymap, part, epi)
 #define GEMV_ONE(mr) if (s.one) GEMV_CASE(mr, true); else GEMV_CASE(mr, false)
     switch (gemv_rows(M)) {
         case 1: GEMV_ONE(1); break;
@@ -3192,9 +3255,10 @@ int dfx_gemm_ex(int wtype, const void * w, int64_t N, int64_t K, const void * ac
     if (M == 0) return DFX_OK;
     hipStream_t st = (hipStream_t)stream;
     const int n = (int)N, k = (int)K, m = (int)M;
-    // the matrix-vector kernels (unless a tile is forced) up to DFX_GEMV_M rows: the same bits as
-    // the matrix-core kernels, whose time does not fall below 32 rows (at four rows, us, against
-    // them: LLaDA-8B gate|up 18 / 25, down 14 / 20, O 7.6 / 10.2, the Q6_K head 99 / 130)
+    // the matrix-vector kernels (unless a tile is forced) up to DFX_GEMV_M rows, where their LDS
+    // holds K: the same bits as the matrix-core kernels, whose time does not fall below 32 rows (at
+    // four rows, us, against them: LLaDA-8B gate|up 18 / 26, down 14 / 21, O 6.9 / 10.3, the Q6_K
+    // head 112 / 126; 16384 x 13568 34 / 52, Q6_K 61 / 63)
     const bool quads = (wtype == DFX_TYPE_Q4_K || wtype == DFX_TYPE_Q6_K) && m <= DFX_GEMV_M && N % 32 == 0 &&
                        !forced_tile(wtype == DFX_TYPE_Q4_K ? 0 : 1).on;
     if (const gemv_shape s = quads ? gemv_launch_shape(wtype, gemv_rows(m), N, K) : gemv_shape{}; s.grid)

@@ -285,16 +285,24 @@ def test_gemm_bias_and_residual_epilogue(gpu):
 GEMV_CASES = [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
               for (N, K) in ((64, 2304), (4608, 3584), (96, 8192), (4096, 12288), (1024, 18944)) for M in (1, 2, 3, 4)]
 GEMV_CASES += [(dfx.TYPE_Q6_K, 152064, 3584, 1), (dfx.TYPE_Q4_K, 37888, 3584, 1)]
+# one pass: few super-blocks to a wave (uneven and single workgroups), and as many threads as there are
+GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
+               for (N, K) in ((32, 256), (544, 768), (1536, 512), (1024, 24576)) for M in (1, 2, 4)]
+GEMV_CASES += [(dfx.TYPE_Q4_K, 1024, 32768, 4), (dfx.TYPE_Q4_K, 1024, 33024, 4)]   # 512 threads; one item more
+# activations staged: 16 or 17 pairs of 9 super-blocks (a second, part-filled pass), more than 64 KB of
+# LDS over one more round of workgroups, and the first K that stays on the matrix cores
+GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
+               for (N, K, Ms) in ((16416, 2304, (1, 2, 3, 4)), (6144, 8192, (4,)), (1056, 17408, (3, 4)), (1056, 17664, (4,)),
+                                  (1056, 34816, (2,)), (1056, 69632, (1,))) for M in Ms]
 
 
 @pytest.mark.parametrize("typ,N,K,M", GEMV_CASES)
 def test_gemv_bit_exact(gpu, typ, N, K, M):
     """At most four rows the matrix-vector kernels run (integer dot products on the int8
-    plane, the exact float order over super-blocks and chunks, a short last chunk at
-    K = 2304 / 3584 / 18944; one, two and four waves per column pair at 1, 2 and 3-5
-    passes of 4096 elements): the oracle's
-    values bit for bit, and the same bits as the
-    matrix-core kernel forced by a tile override."""
+    plane, the exact float order over super-blocks and chunks, short last chunks, a lane per
+    output and chunk from three chunks on): the oracle's values bit for bit, and the same bits as the
+    matrix-core kernel forced by a tile override.  Workgroups of one pass (most of the narrow
+    matrices here) and of several with the activations staged."""
     raw = quant(typ, N, K)
     X = rng.standard_normal((M, K)).astype(np.float32)
     got = gpu_gemm(typ, raw, N, K, X)
