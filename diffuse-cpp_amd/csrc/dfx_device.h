@@ -58,9 +58,27 @@ __device__ __forceinline__ float wave_sum(float v) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
     return v;
 }
+// The xor butterfly 32, 16, 8, 4, 2, 1 in the VALU: v_permlane32_swap / 16_swap pair the halves and
+// the rows of 16, row rotations by 8 and 4 are the xors once the levels above have made the row
+// periodic, quad permutes the last two.
+template <int CTRL> __device__ __forceinline__ double dpp_sum(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, true);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
+    return v + __builtin_bit_cast(double, (uint64_t)h << 32 | l);
+}
 __device__ __forceinline__ double wave_sum_d(double v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+    auto pair = [](uint32_t l0, uint32_t h0, uint32_t l1, uint32_t h1) {
+        return __builtin_bit_cast(double, (uint64_t)h0 << 32 | l0) + __builtin_bit_cast(double, (uint64_t)h1 << 32 | l1);
+    };
+    uint64_t b = __builtin_bit_cast(uint64_t, v);
+    auto l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    b = __builtin_bit_cast(uint64_t, pair(l[0], h[0], l[1], h[1]));
+    l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    v = pair(l[0], h[0], l[1], h[1]);
+    return dpp_sum<0xB1>(dpp_sum<0x4E>(dpp_sum<0x124>(dpp_sum<0x128>(v))));   // row_ror 8, 4; quad_perm
 }
 
 // ---- converted activations (the GEMM input) ----

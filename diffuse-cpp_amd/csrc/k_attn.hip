@@ -539,6 +539,11 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
 // of four MFMAs as they are, the A operands one 16-byte load of the transposed value cache per
 // 16 value columns; the waves' f64 sums are added in a fixed order through LDS.
 // Key tiles that no row of the query tile sees are not visited.
+// NT = 1 (head size 128): with up to eight key tiles most of phase 3's f64 partial outputs are one
+// tile's, or nothing, and adding them through 128 KB of LDS outweighs the product.  The waves'
+// probabilities go through LDS instead (8 KB, each lane's four as they are), and wave w makes the 16
+// value columns w over all key tiles: 16 rows of 32 heads over 16 keys 6.4 us instead of 7.7, 32 rows
+// over 32 keys 7.1 / 7.8, 64 over 96 9.5 / 10.5, 128 over 128 10.6 / 11.2.
 // Bound by the f64 matrix cores (62 TFLOP/s measured on a large product): 4096 keys, 512 causal
 // rows of 28 heads 620 us (floor 455) against 1704 when the scores were recomputed in three
 // passes; 768 keys and rows of 32 heads 192 us (floor 156) against 222 with scores in LDS, whose
@@ -550,8 +555,9 @@ k_attn_keep(const float * __restrict__ q, const float * __restrict__ kc, const f
             int M, int n_keys, int H, int Hkv, int q_tiles, int q_pos0, int window, float * __restrict__ out) {
 #pragma clang fp contract(off)
     constexpr int NW = 8, SS = HD / 16, CT = HD / 16;
-    constexpr int RW = WPE == 2 ? NW : NW / 2;       // waves whose partial outputs are in LDS at once
-    __shared__ __attribute__((aligned(16))) double R[RW * HD * 16];   // query [SS][2][64][2], then partial outputs
+    constexpr bool COLS = NT == 1;                   // one tile per wave: phase 3 by column tiles
+    constexpr int RW = COLS ? 1 : WPE == 2 ? NW : NW / 2;   // waves whose partial outputs are in LDS at once
+    __shared__ __attribute__((aligned(16))) double R[RW * HD * 16];   // query [SS][2][64][2], then partial outputs (COLS: P)
     __shared__ float red_f[NW][16];
     __shared__ double red_d[NW][16];
     // unit u = (head, query tile), heads of one KV head adjacent; XCD x (= workgroup mod 8) takes
@@ -638,7 +644,14 @@ k_attn_keep(const float * __restrict__ q, const float * __restrict__ kc, const f
 #pragma unroll
         for (int c = 0; c < HC; c++) vf[hf][c] = *(const f32x4 *)(vb + (int64_t)16 * (HC * hf + c) * v_ld + 16 * t);
     };
-    load_v(lo, min(t0 + wv, t1 - 1));
+    f32x4 vc[NW];                                     // COLS: this wave's column tile, every key tile
+    if constexpr (COLS) {
+        static_assert(CT == NW, "a column tile per wave");
+#pragma unroll
+        for (int j = 0; j < NW; j++) vc[j] = *(const f32x4 *)(vb + (int64_t)16 * wv * v_ld + 16 * min(t0 + j, t1 - 1));
+    } else {
+        load_v(lo, min(t0 + wv, t1 - 1));
+    }
 
     // ---- phase 2
     float mx = -INFINITY;
@@ -672,6 +685,27 @@ k_attn_keep(const float * __restrict__ q, const float * __restrict__ kc, const f
     const float inv = (float)(1.0 / sum);
 
     // ---- phase 3
+    if constexpr (COLS) {
+        f32x4 * P = (f32x4 *)R;                      // every wave is past phase 1
+        if (t0 + wv < t1) P[wv * 64 + lane] = f32x4{sc[0][0] * inv, sc[0][1] * inv, sc[0][2] * inv, sc[0][3] * inv};
+        __syncthreads();
+        double4v o[2] = {0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < NW; j++)
+            if (t0 + j < t1) {
+                const f32x4 p = P[j * 64 + lane];
+                const int n = 16 * (t0 + j) + 4 * lg;
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    o[j & 1] = mfma_f64((double)(n + i < n_keys ? vc[j][i] : 0.0f), (double)p[i], o[j & 1]);
+            }
+        const int row = q0 + li;
+        if (row < M)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                out[((int64_t)row * H + h) * HD + 16 * wv + 4 * i + lg] = (float)(o[0][i] + o[1][i]);
+        return;
+    }
     double4v o[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ct++) o[ct] = 0.0;
@@ -734,15 +768,10 @@ k_attn_keep(const float * __restrict__ q, const float * __restrict__ kc, const f
 // are added at the end and rounded to float once.  Only the f64 summation order differs from the
 // oracle's (as in the matrix-core kernels): a float result differs where two orders straddle a
 // rounding boundary.  Bound by the latency of its loads and one CU's bandwidth: one row of 28
-// heads 7.4 us over 192 keys, 19.9 over 1024, 73.9 over 4096 (four waves and a thread per output
+// heads 7.0 us over 192 keys, 20.1 over 1024, 73.9 over 4096 (four waves and a thread per output
 // dimension and key range, each lane reading its own value row: 10.2, 33.9; the matrix-core tile
-// 582).
-template <int CTRL> __device__ __forceinline__ double dpp_sum(double v) {
-    const uint64_t b = __builtin_bit_cast(uint64_t, v);
-    const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, true);
-    const uint32_t h = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
-    return v + __builtin_bit_cast(double, (uint64_t)h << 32 | l);
-}
+// 582).  Over few keys the f64 sum across the wave counts: in the VALU instead of LDS permutes, one
+// row of 32 heads over 48 keys 5.9 us instead of 6.2.
 #define ROWS_MAX_KEYS 32768
 template <int HD>
 __global__ void __launch_bounds__(8 * HD) k_attn_rows(const float * __restrict__ q, const float * __restrict__ kc,
@@ -956,7 +985,8 @@ static int attn_exact(const float * q, const float * kc, const float * vt, int64
     hipLaunchKernelGGL((k_attn_keep<HD, NT, WPE>), g, dim3(512), 0, st, q, kc, vt, v_ld, M, n_keys, H, Hkv, q_tiles,   \
                        q_pos0, window, out)
         if (hd == 128) {
-            if (two && nt <= 2) KEEP(128, 2, 4);
+            if (nt <= 1) KEEP(128, 1, 4);
+            else if (two && nt <= 2) KEEP(128, 2, 4);
             else if (two && nt <= 3) KEEP(128, 3, 4);
             else if (two && nt <= 4) KEEP(128, 4, 4);
             else if (two && nt <= 6) KEEP(128, 6, 4);

@@ -591,11 +591,14 @@ def test_attention_exact_matches_oracle_and_f64(gpu, M, n_keys, H, Hkv, hd):
 
 
 # Edges of the forms behind dfx_attention_causal: one workgroup per row and head up to as many as
-# CUs (8 rows of 32 heads), then 16-row tiles with 2, 3, 4, 6, 8, 16 or 32 key tiles per wave, one
-# or two workgroups per CU, then the recomputing form above 4096 visible keys.
+# CUs (8 rows of 32 heads), then 16-row tiles with up to eight key tiles in all (head size 128), or 2,
+# 3, 4, 6, 8, 16 or 32 key tiles per wave, one or two workgroups per CU, then the recomputing form above
+# 4096 visible keys.
 @pytest.mark.parametrize("M,n_keys,H,Hkv,hd,window", [
     (8, 33, 32, 4, 128, 0), (9, 33, 32, 4, 128, 0), (1, 1, 3, 1, 128, 0), (2, 1025, 5, 5, 64, 0),
     (3, 4100, 2, 2, 128, 70), (5, 300, 4, 2, 64, 29),
+    (16, 16, 32, 32, 128, 0), (33, 33, 28, 4, 128, 0), (97, 128, 32, 8, 128, 0), (97, 129, 32, 8, 128, 0),
+    (300, 300, 2, 2, 128, 60),
     (150, 256, 28, 4, 128, 0), (150, 257, 28, 4, 128, 0), (150, 385, 28, 4, 128, 0), (150, 513, 28, 4, 128, 0),
     (150, 769, 28, 4, 128, 0), (270, 513, 17, 17, 64, 0), (270, 1025, 17, 17, 64, 0), (270, 1030, 17, 17, 64, 100),
     (130, 512, 2, 1, 128, 0), (130, 513, 2, 1, 128, 0), (130, 1025, 2, 1, 128, 0), (130, 2049, 2, 1, 128, 0),
