@@ -204,8 +204,8 @@ int dfx_rope_store(const float * qkv, const int32_t * pos, int64_t M, int H, int
 /* Bidirectional attention, no mask (src/diffuse-graph.cpp:97-119 / 528-553):
  * out[m][h*hd + j] = sum_n softmax_n(q_m . k_n / sqrt(hd)) * v_n[j], keys 0..n_keys-1
  * of the cache (kc[n][Hkv][hd], vt[Hkv][hd][v_ld], n_keys <= v_ld, v_ld a multiple of
- * 16), query head h reads KV head h / (H/Hkv).  Any number of keys: score rows that do not
- * fit the LDS are recomputed instead of stored. */
+ * 16), query head h reads KV head h / (H/Hkv).  Any number of keys: a row's scores stay on the chip
+ * up to 4096 visible keys (32768 where M x H is at most the CU count), beyond they are recomputed. */
 int dfx_attention(const float * q, const float * kc, const float * vt, int64_t v_ld, int64_t M, int64_t n_keys,
                   int H, int Hkv, int hd, float * out, void * stream);   /* mode DFX_ATTN_EXACT */
 

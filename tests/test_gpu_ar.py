@@ -44,7 +44,7 @@ def _same(got, ref, scheme, what):
 CAUSAL_SHAPES = [  # M, n_keys, q_pos0, window, H, Hkv, hd
     (7, 30, 23, 0, 4, 2, 128), (7, 30, 23, 5, 4, 2, 128), (1, 300, 299, 0, 8, 8, 64), (33, 33, 0, 0, 4, 4, 128),
     (33, 33, 0, 8, 6, 3, 64), (16, 100, 40, 1, 2, 2, 128),
-    # score rows longer than the LDS holds: the three-pass kernel
+    # many keys: a workgroup per row and head
     (3, 3000, 2997, 0, 2, 1, 128), (20, 2800, 2700, 700, 4, 2, 64)]
 
 
@@ -71,11 +71,11 @@ def test_attention_causal_matches_oracle(gpu, M, n_keys, q_pos0, window, H, Hkv,
 
 @pytest.mark.parametrize("M,n_keys,q_pos0,window,H,Hkv,hd", [
     (1, 192, 191, 0, 28, 4, 128),      # Dream-7B decode: one row, GQA 28 / 4
-    (1, 1024, 1023, 0, 8, 2, 64),      # the most keys of the few-row kernel
+    (1, 1024, 1023, 0, 8, 2, 64),
     (4, 700, 696, 100, 4, 1, 128),     # four rows with a window
     (2, 65, -1, 0, 4, 4, 128)])        # bidirectional (no mask)
 def test_attention_few_rows_matches_oracle(gpu, M, n_keys, q_pos0, window, H, Hkv, hd):
-    """At most 4 query rows and 1024 keys (decoding): one workgroup per row and head.  The same
+    """Few query rows (decoding; rows x heads up to the CU count): one workgroup per row and head.  The same
     f64 sums of exact products as the oracle in another order: equal floats except where two
     orders straddle an f32 rounding boundary (at most one ulp, rare)."""
     rng = np.random.default_rng(M * 7 + n_keys)
@@ -174,7 +174,7 @@ def test_ar_prefill_and_decode_match_oracle(gpu, ar_models, arch, scheme, window
 
 
 def test_ar_long_context(gpu, ar_models):
-    """2600-position prompt (score rows past the LDS: the three-pass attention), then two
+    """2600-position prompt (21 key tiles per wave of the exact attention), then two
     decodes, full causal and with a window.  Over this many rows a one-ulp attention
     difference (two f64 summation orders) can move one int8 activation step, so the check is
     the logits bar plus at least 99% of the rows bit-identical."""

@@ -538,8 +538,9 @@ def test_rope_store_matches_oracle(gpu, M, H, Hkv, hd, n_ctx):
 ATTN_SHAPES = [(288, 288, 32, 32, 128), (50, 288, 32, 32, 128), (128, 128, 28, 4, 128), (7, 768, 8, 2, 64),
                (3, 2000, 4, 4, 128), (2, 3000, 2, 1, 128), (17, 1, 4, 4, 128), (33, 21, 4, 2, 64),
                (768, 768, 32, 32, 128), (256, 768, 32, 32, 128), (65, 97, 6, 3, 64), (1, 33, 2, 2, 128),
-               # score rows longer than the LDS holds (three-pass form), past 16k keys, both head sizes
-               (19, 40000, 2, 1, 128), (5, 9000, 4, 2, 64)]
+               # more than 4096 keys: recomputed in three passes where rows x heads is more than the CUs or
+               # past 32768 keys, both head sizes; else a workgroup per row and head
+               (19, 40000, 2, 1, 128), (70, 4200, 4, 2, 64), (5, 9000, 4, 2, 64)]
 
 
 def attention_case(M, n_keys, H, Hkv, hd, mode):
@@ -568,8 +569,8 @@ def attention_case(M, n_keys, H, Hkv, hd, mode):
 @pytest.mark.parametrize("M,n_keys,H,Hkv,hd", ATTN_SHAPES)
 def test_attention_exact_matches_oracle_and_f64(gpu, M, n_keys, H, Hkv, hd):
     """DFX_ATTN_EXACT: bit-exact with the oracle (f64 accumulation of exact products,
-    correctly rounded exp), and within 1e-6 of an independent f64 evaluation.  Covers
-    the 16-row matrix-core kernel (score rows in LDS) and the VALU kernel (3000 keys)."""
+    correctly rounded exp), and within 1e-6 of an independent f64 evaluation: the 16-row
+    matrix-core kernels (scores in registers, or recomputed) and the few-row kernel."""
     got, ref, q, k, v = attention_case(M, n_keys, H, Hkv, hd, dfx.ATTN_EXACT)
     assert rel_l2(got, ref) < 1e-6
     exact = O.attention(q, k, v)
@@ -603,7 +604,12 @@ def test_attention_exact_matches_oracle_and_f64(gpu, M, n_keys, H, Hkv, hd):
     (150, 769, 28, 4, 128, 0), (270, 513, 17, 17, 64, 0), (270, 1025, 17, 17, 64, 0), (270, 1030, 17, 17, 64, 100),
     (130, 512, 2, 1, 128, 0), (130, 513, 2, 1, 128, 0), (130, 1025, 2, 1, 128, 0), (130, 2049, 2, 1, 128, 0),
     (130, 4096, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 200), (130, 520, 2, 1, 64, 16),
-    (130, 1030, 2, 2, 64, 0), (130, 2060, 2, 2, 64, 0)])
+    (130, 1030, 2, 2, 64, 0), (130, 2060, 2, 2, 64, 0),
+    # recomputed at head size 64, and from a first key tile past 0 with a window above 4096, at both
+    (130, 4300, 2, 1, 64, 0), (130, 4500, 2, 2, 64, 4200), (130, 4500, 2, 1, 128, 4200),
+    # a workgroup per row and head over as many keys as the LDS takes, and one key more (recomputed)
+    (1, 20000, 2, 1, 128, 0), (1, 32768, 2, 1, 128, 0), (2, 32768, 2, 2, 64, 30000), (1, 32769, 2, 1, 128, 0),
+    (2, 32769, 2, 2, 64, 0)])
 def test_attention_causal_matches_f64(gpu, M, n_keys, H, Hkv, hd, window):
     """Against float64 with the mask.  Scores, probabilities and outputs are rounded to f32 once each
     (scores of up to about 40 in size move their exponentials by 40 * 2^-24): 4e-6 of the result.
