@@ -544,7 +544,8 @@ __global__ void __launch_bounds__(256) k_attn_long(const float * __restrict__ q,
 // probabilities go through LDS instead (8 KB, each lane's four as they are), and wave w makes the 16
 // value columns w over all key tiles: 16 rows of 32 heads over 16 keys 6.4 us instead of 7.7, 32 rows
 // over 32 keys 7.1 / 7.8, 64 over 96 9.5 / 10.5, 128 over 128 10.6 / 11.2.
-// Bound by the f64 matrix cores (62 TFLOP/s measured on a large product): 4096 keys, 512 causal
+// Bound by the f64 matrix cores (62 TFLOP/s measured on a large product; busy 56-58 % of the time
+// here, and waves queue for them 60 % of theirs): 4096 keys, 512 causal
 // rows of 28 heads 620 us (floor 455) against 1704 when the scores were recomputed in three
 // passes; 768 keys and rows of 32 heads 192 us (floor 156) against 222 with scores in LDS, whose
 // softmax read and wrote them three times; 288 by 288 46 against 52.  WPE waves per SIMD: 2 (one
