@@ -313,9 +313,10 @@ def test_gemv_bit_exact(gpu, typ, N, K, M):
     assert np.array_equal(got.view(np.uint32), mfma.view(np.uint32))
 
 
-def test_gemv_epilogues_and_row_map(gpu):
-    """Bias, in-place residual and a row map through the matrix-vector kernel."""
-    typ, N, K, M = dfx.TYPE_Q4_K, 1024, 4096, 3
+@pytest.mark.parametrize("typ,N,K,M", [(dfx.TYPE_Q4_K, 1024, 4096, 3), (dfx.TYPE_Q4_K, 16416, 2304, 4),
+                                       (dfx.TYPE_Q6_K, 16416, 2304, 1)])
+def test_gemv_epilogues_and_row_map(gpu, typ, N, K, M):
+    """Bias and in-place residual through the matrix-vector kernel, in one pass and with the activations staged."""
     raw = quant(typ, N, K)
     X = rng.standard_normal((M, K)).astype(np.float32)
     w = to_device_weights(typ, raw, N, K)
@@ -362,6 +363,7 @@ def oracle_swiglu(g, u):
     (dfx.TYPE_Q4_K, 1024, 4096, 130, "w"), (dfx.TYPE_Q4_K, 1024, 4096, 130, "ws"),
     (dfx.TYPE_Q4_K, 1024, 3584, 150, "w3"), (dfx.TYPE_Q4_K, 512, 12288, 5, "1x1x4s"),
     (dfx.TYPE_Q4_K, 2048, 4096, 1, None), (dfx.TYPE_Q4_K, 1024, 4096, 4, None), (dfx.TYPE_Q6_K, 512, 4096, 2, None),
+    (dfx.TYPE_Q4_K, 8208, 2304, 3, None), (dfx.TYPE_Q6_K, 8208, 2304, 2, None),   # matrix-vector, activations staged
     (dfx.TYPE_Q4_K, 2688, 3584, 24, None),   # wide, few rows: two-wave tiles, split K, SwiGLU in the reduction
     (dfx.TYPE_Q6_K, 512, 12288, 40, "2x1s"), (dfx.TYPE_Q4_K, 512, 12288, 40, "ks"), (dfx.TYPE_Q4_K, 512, 3584, 70, "k"), (dfx.TYPE_Q4_K, 768, 4096, 50, "k4"),
     (dfx.TYPE_Q6_K, 512, 4096, 66, "2x1n"), (dfx.TYPE_Q8_0, 512, 4096, 33, None),
@@ -425,6 +427,7 @@ def rope_row_order(H, Hkv, hd):
     (dfx.TYPE_Q4_K, 4, 2, 128, 4096, 200, "ws", False), (dfx.TYPE_Q4_K, 8, 8, 128, 4096, 3, None, False),
     (dfx.TYPE_Q4_K, 4, 2, 128, 3584, 1, None, True), (dfx.TYPE_Q6_K, 4, 4, 64, 4096, 2, None, False),
     (dfx.TYPE_Q4_K, 4, 2, 128, 3584, 50, "ks", True), (dfx.TYPE_Q4_K, 6, 2, 64, 4096, 40, "k", True), (dfx.TYPE_Q4_K, 4, 2, 128, 4096, 74, "k2s", True),
+    (dfx.TYPE_Q4_K, 32, 32, 128, 3584, 2, None, True), (dfx.TYPE_Q6_K, 32, 32, 128, 3584, 1, None, False),   # staged
     (dfx.TYPE_Q6_K, 4, 2, 128, 4096, 66, "2x1s", True), (dfx.TYPE_Q6_K, 4, 4, 64, 2048, 100, "2x1n", False),
     (dfx.TYPE_Q8_0, 4, 2, 128, 2048, 33, None, True), (dfx.TYPE_F16, 4, 1, 128, 2048, 45, None, True),
     (dfx.TYPE_F16, 32, 32, 128, 256, 300, None, True),
