@@ -1866,8 +1866,9 @@ k_gemm_f16(const uint8_t * __restrict__ W, int N, int K, const half_t * __restri
 // What bounds it: from cache the loop runs at the matrix cores' rate (0.52 us a step of the 192 x 384
 // tile, 0.48 us of MFMAs at 2.4 GHz); with weights from HBM at 0.84 us, a CU's outstanding misses
 // (about 64 KB) over their latency, which more copies ahead, or lines fetched into L2 ahead of the
-// copies, do not change (10 % slower); the matrix cores are busy 42-45 % of the time then.  LLaDA-8B at 768 rows, cold weights, us a call, before -> after:
-// gate|up 244 -> 154, down 129 -> 97, Q|K|V 141 -> 92, O 53 -> 48; the whole FFN block 386 -> 274.
+// copies, do not change (10 % slower); the matrix cores are busy 42-45 % of the time then.  LLaDA-8B
+// at 768 rows, cold weights, us a call, before -> after: gate|up 244 -> 154, down 129 -> 97, Q|K|V
+// 141 -> 92, O 53 -> 48; the whole FFN block 386 -> 274.
 template <int WM, int WN, int TM, int TN>
 __global__ void __launch_bounds__(64 * WM * WN, 2)
 k_gemm_f16_w(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ A, int M,
