@@ -2954,13 +2954,17 @@ template <int WT> struct gemv_raw;
 template <> struct gemv_raw<DFX_TYPE_Q4_K> { u32x4 h[2], q[2][2]; };
 template <> struct gemv_raw<DFX_TYPE_Q6_K> { u32x4 la[2], lb[2], qh[2], sc[2]; uint32_t d[2]; };
 
-template <int WT, int MR, bool ONE>
+// GEMV_STAGED: the activations in LDS; GEMV_ONE: straight from memory, a workgroup's items in one pass;
+// GEMV_PASSES: straight from memory, in several.
+enum gemv_form { GEMV_STAGED, GEMV_ONE, GEMV_PASSES };
+
+template <int WT, int MR, gemv_form FORM>
 __global__ void __launch_bounds__(gemv_threads(WT, MR)) __attribute__((amdgpu_waves_per_eu(gemv_threads(WT, MR) / 128)))
 k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict__ act, int M,
        const float * __restrict__ bias, const float * res, float * Y, int64_t ldy, const int32_t * __restrict__ ymap,
        gemv_part part, dfx_epi epi) {
 #pragma clang fp contract(off)
-    constexpr bool Q4 = WT == DFX_TYPE_Q4_K;
+    constexpr bool Q4 = WT == DFX_TYPE_Q4_K, DIRECT = FORM != GEMV_STAGED;
     constexpr int SB = Q4 ? SB_Q4_K : SB_Q6_K;
     extern __shared__ __attribute__((aligned(16))) uint8_t gemv_lds[];
     const int tid = threadIdx.x, g = tid & 3;
@@ -2972,7 +2976,7 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
     auto pair_of = [&](int t) __attribute__((always_inline)) -> int {
         return (int)__umulhi(2 * (uint32_t)t + 1, part.inv_nsb);
     };
-    const int a_bytes = ONE ? 0 : MR * K, b_bytes = ONE ? 0 : MR * nsb * 32;
+    const int a_bytes = DIRECT ? 0 : MR * K, b_bytes = DIRECT ? 0 : MR * nsb * 32;
     u32x4 * as = (u32x4 *)gemv_lds;                           // [MR][4][nsb * 4]: piece i of group g
     uint2 * bs = (uint2 *)(gemv_lds + a_bytes);               // [MR][nsb * 4]: the group's sums
     float * xs = (float *)(gemv_lds + a_bytes + b_bytes);     // [MR][nsb][ncol]
@@ -3023,16 +3027,16 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
             }
         }
     };
-    // ONE: the lane's activations and sums, requested with its weights
-    u32x4 a1[ONE ? MR : 1][4];
-    uint2 b1[ONE ? MR : 1];
+    // DIRECT: the lane's activations and sums, requested with its weights
+    u32x4 a1[DIRECT ? MR : 1][4];
+    uint2 b1[DIRECT ? MR : 1];
     auto compute = [&](int t, const gemv_raw<WT> & r) __attribute__((always_inline)) {
         const int pl = pair_of(t), sb = t - pl * nsb;
 #pragma unroll
         for (int m = 0; m < MR; m++) {
             u32x4 a[4];
             uint2 b;
-            if constexpr (ONE) {
+            if constexpr (DIRECT) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) a[i] = a1[m][i];
                 b = b1[m];
@@ -3088,7 +3092,7 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
     int t = tid >> 2;
     load(t, r0);
     float d1[MR];
-    if constexpr (ONE) {
+    if constexpr (DIRECT) {
         const int tc = min(t, items - 1), sb = tc - pair_of(tc) * nsb;
 #pragma unroll
         for (int m = 0; m < MR; m++) {
@@ -3119,11 +3123,27 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
             for (int m = 0; m < MR; m++) ds[m * nsb + sb] = ad[(int64_t)sb * Lay.mq + min(m, M - 1)];
     }
     // (a quad's four lanes share its items, so quad_sum sees all of them or none)
-    if constexpr (ONE) {
+    if constexpr (DIRECT) {
         if (t < items) compute(t, r0);
         if (tid < nsb)
 #pragma unroll
             for (int m = 0; m < MR; m++) ds[m * nsb + tid] = d1[m];
+        if constexpr (FORM == GEMV_PASSES) {
+            for (int sb = tid + (int)blockDim.x; sb < nsb; sb += (int)blockDim.x)
+#pragma unroll
+                for (int m = 0; m < MR; m++) ds[m * nsb + sb] = ad[(int64_t)sb * Lay.mq + min(m, M - 1)];
+            for (t += T4; t < items; t += T4) {
+                load(t, r0);
+                const int sb = t - pair_of(t) * nsb;
+#pragma unroll
+                for (int m = 0; m < MR; m++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) a1[m][i] = piece(m, sb, g, i);
+                    b1[m] = sums(m, sb, g);
+                }
+                compute(t, r0);
+            }
+        }
     } else {
         __syncthreads();
         for (; t < items; t += 2 * T4) {
@@ -3168,18 +3188,21 @@ k_gemv(const uint8_t * __restrict__ W, int N, int K, const uint8_t * __restrict_
     }
 }
 
-// Launch of a matrix-vector call.  ONE where a workgroup's items fit one pass over two workgroups
+// Launch of a matrix-vector call.  GEMV_ONE where a workgroup's items fit one pass over two workgroups
 // per CU, each of them filling a wave (16 / nsb pairs) if there are so few (1536 x 512: 96 workgroups
 // 3.1 us, 512 of a quarter of a wave 3.6), with as many threads as the items take: activations
 // straight from global memory then, beside the weights.  Else the activations are staged, in up to
 // half of a CU's 160 KB; where the outputs' x needs more workgroups than two per CU, whole rounds of
-// them (N = 28672, K = 8192 at four rows: 1024 instead of 531, 33 us instead of 44).  grid = 0: one pair of
-// columns would not fit (K beyond 17 k at three or four rows, 34 k at two, 69 k at one).
+// them (N = 28672, K = 8192 at four rows: 1024 instead of 531, 33 us instead of 44).  Where the
+// staged activations and one pair would not fit (K beyond 17 k at three or four rows, 34 k at two, 69 k
+// at one): one or two rows take their activations from memory in every pass (1024 x 131072, one row
+// 26 us, the matrix cores 46; 4096 x 36864, two rows 29 / 45), more stay on the matrix cores (8192 x 28672,
+// four rows 58 us against 80 in passes): grid = 0.
 constexpr int64_t GEMV_LDS = 80 * 1024;
 struct gemv_shape {
     int grid, threads;
     size_t lds;
-    bool one;
+    gemv_form form;
 };
 static gemv_shape gemv_launch_shape(int wtype, int mr, int64_t N, int64_t K) {
     const int64_t nsb = K / 256, pairs = N / 2, per_pair = mr * nsb * 8, slots = 2 * device_cu_count();
@@ -3187,12 +3210,17 @@ static gemv_shape gemv_launch_shape(int wtype, int mr, int64_t N, int64_t K) {
     if (4 * ((pairs + slots - 1) / slots) * nsb <= threads) {
         const int64_t fill = std::max<int64_t>(1, 16 / nsb), g = std::min((pairs + fill - 1) / fill, slots);
         const int64_t most = (pairs + g - 1) / g;
-        return {(int)g, (int)((4 * most * nsb + 63) / 64 * 64), (size_t)(mr * nsb * 4 + most * per_pair), true};
+        return {(int)g, (int)((4 * most * nsb + 63) / 64 * 64), (size_t)(mr * nsb * 4 + most * per_pair), GEMV_ONE};
     }
     const int64_t fixed = mr * (K + nsb * 36), room = (GEMV_LDS - fixed) / per_pair;
-    if (GEMV_LDS < fixed + per_pair) return {0, 0, 0, false};
+    if (GEMV_LDS < fixed + per_pair) {
+        const int64_t fit = (GEMV_LDS - mr * nsb * 4) / per_pair;
+        if (mr > 2 || fit < 1) return {};
+        const int64_t g = std::min(pairs, (pairs + fit * slots - 1) / (fit * slots) * slots);
+        return {(int)g, threads, (size_t)(mr * nsb * 4 + (pairs + g - 1) / g * per_pair), GEMV_PASSES};
+    }
     const int64_t g = std::min(pairs, (pairs + room * slots - 1) / (room * slots) * slots);
-    return {(int)g, threads, (size_t)(fixed + (pairs + g - 1) / g * per_pair), false};
+    return {(int)g, threads, (size_t)(fixed + (pairs + g - 1) / g * per_pair), GEMV_STAGED};
 }
 static int gemv_rows(int M) { return M <= 2 ? M : DFX_GEMV_M; }
 
@@ -3203,15 +3231,17 @@ static int launch_gemv(const void * w, int N, int K, const void * act, int M, co
     const uint8_t * A = (const uint8_t *)act;
     const uint32_t nsb = (uint32_t)(K / 256);
     const gemv_part part = {N / 2 / s.grid, N / 2 % s.grid, (0x80000000u + nsb - 1) / nsb};
-#define GEMV_CASE(mr, one) hipLaunchKernelGGL((k_gemv<WT, mr, one>), dim3((unsigned)s.grid), dim3((unsigned)s.threads), \
-                                              s.lds, st, W, N, K, A, M, bias, res, y, ldy, ymap, part, epi)
-#define GEMV_ONE(mr) if (s.one) GEMV_CASE(mr, true); else GEMV_CASE(mr, false)
+#define GEMV_CASE(mr, form) hipLaunchKernelGGL((k_gemv<WT, mr, form>), dim3((unsigned)s.grid), dim3((unsigned)s.threads), \
+                                               s.lds, st, W, N, K, A, M, bias, res, y, ldy, ymap, part, epi)
+#define GEMV_FORM(mr) if (s.form == GEMV_ONE) GEMV_CASE(mr, GEMV_ONE); else GEMV_CASE(mr, GEMV_STAGED)
+#define GEMV_FORM3(mr) if (s.form == GEMV_PASSES) GEMV_CASE(mr, GEMV_PASSES); else GEMV_FORM(mr)
     switch (gemv_rows(M)) {
-        case 1: GEMV_ONE(1); break;
-        case 2: GEMV_ONE(2); break;
-        default: GEMV_ONE(4); break;
+        case 1: GEMV_FORM3(1); break;
+        case 2: GEMV_FORM3(2); break;
+        default: GEMV_FORM(4); break;
     }
-#undef GEMV_ONE
+#undef GEMV_FORM3
+#undef GEMV_FORM
 #undef GEMV_CASE
     DFX_CHECK_LAUNCH("dfx_gemm (matrix-vector)");
     return DFX_OK;

@@ -113,8 +113,8 @@ int dfx_swiglu_convert(int wtype, const float * gu, int64_t M, int64_t F, void *
 /* GEMM (src/diffuse-graph.cpp:61-63, 122, 136-140, 154):
  *   y[m][n] = sum_k x[m][k] * W[n][k]  (+ bias[n])  (+ residual[m][n])
  * on the matrix cores, or for up to four rows of Q4_K / Q6_K weights on integer dot products over
- * the int8 copy that the conversions keep for them (K up to 17 k at three or four rows, 34 k at two,
- * 69 k at one, more over few columns: what the LDS holds; longer rows stay on the matrix cores).
+ * the int8 copy that the conversions keep for them (three or four rows of K beyond 17 k, what the LDS
+ * holds, stay on the matrix cores unless the columns are few).
  * act: the converted activations of x (dfx_*_convert with the same wtype and the same M: the
  * layout depends on M);
  * W: device-layout [N][K]; y f32 [M][N].  For Q4_K / Q6_K / Q8_0 the result

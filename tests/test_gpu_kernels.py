@@ -294,6 +294,10 @@ GEMV_CASES += [(dfx.TYPE_Q4_K, 1024, 32768, 4), (dfx.TYPE_Q4_K, 1024, 33024, 4)]
 GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
                for (N, K, Ms) in ((16416, 2304, (1, 2, 3, 4)), (6144, 8192, (4,)), (1056, 17408, (3, 4)), (1056, 17664, (4,)),
                                   (1056, 34816, (2,)), (1056, 69632, (1,))) for M in Ms]
+# one or two rows that cannot be staged: several passes from memory, the last part-filled; more
+# super-blocks than threads
+GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
+               for (N, K, M) in ((1056, 35072, 2), (1056, 69888, 1), (64, 131072, 1), (64, 131072, 2))]
 
 
 @pytest.mark.parametrize("typ,N,K,M", GEMV_CASES)
@@ -302,7 +306,7 @@ def test_gemv_bit_exact(gpu, typ, N, K, M):
     plane, the exact float order over super-blocks and chunks, short last chunks, a lane per
     output and chunk from three chunks on): the oracle's values bit for bit, and the same bits as the
     matrix-core kernel forced by a tile override.  Workgroups of one pass (most of the narrow
-    matrices here) and of several with the activations staged."""
+    matrices here) and of several, with the activations staged or from memory."""
     raw = quant(typ, N, K)
     X = rng.standard_normal((M, K)).astype(np.float32)
     got = gpu_gemm(typ, raw, N, K, X)
